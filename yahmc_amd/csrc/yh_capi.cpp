@@ -405,8 +405,9 @@ int yh_create(const yh_lattice* lat, yh_ctx** out) {
     e = hipHostMalloc((void**)&c->sc_ring, Ctx::SC_RING * sizeof(SolverScalars), hipHostMallocDefault);
   for (int i = 0; i < Ctx::SC_RING && e == hipSuccess; i++)
     e = hipEventCreateWithFlags(&c->ev_ring[i], hipEventDisableTiming);
-  if (e == hipSuccess) e = hipMalloc(&c->fund, sizeof(double) * 4 * (size_t)V * 2 * lat->nc * lat->nc);
-  if (e == hipSuccess) e = hipMalloc(&c->tab, sizeof(double2) * (TAB_BASIS + TAB_ITR + TAB_ITF));
+  if (e == hipSuccess) e = hipMalloc(&c->fund, sizeof(double2) * 8 * (size_t)c->g.VHpad * lat->nc * lat->nc);
+  if (e == hipSuccess) e = hipMalloc(&c->fund_aos, sizeof(double) * 4 * (size_t)V * 2 * lat->nc * lat->nc);
+  if (e == hipSuccess) e = hipMalloc(&c->tab, sizeof(double2) * (TAB_BASIS + TAB_ITR));
   if (e != hipSuccess) {
     set_error(std::string("context allocation: ") + hipGetErrorString(e));
     yh_destroy(c);
@@ -414,11 +415,9 @@ int yh_create(const yh_lattice* lat, yh_ctx** out) {
   }
   c->tab_basis = c->tab;
   c->tab_itr = c->tab + TAB_BASIS;
-  c->tab_itf = c->tab + TAB_BASIS + TAB_ITR;
   int rc = noalloc_init(c->device);
   if (!rc) rc = gauge_init_basis(c);
   if (!rc) rc = force_init_constants(c);
-  if (!rc) rc = md_init_constants(c);
   if (!rc) rc = meson_init_tables();
   if (rc) { yh_destroy(c); return rc; }
   *out = c;
@@ -443,6 +442,7 @@ int yh_destroy(yh_ctx* c) {
   for (int i = 4; i < 6; i++)
     if (c->tmp[i]) { (void)hipFree(c->tmp[i]->mem); delete static_cast<yh_field*>(c->tmp[i]); }
   if (c->fund) (void)hipFree(c->fund);
+  if (c->fund_aos) (void)hipFree(c->fund_aos);
   if (c->tab) (void)hipFree(c->tab);
   if (c->logdet_site) (void)hipFree(c->logdet_site);
   if (c->mom) (void)hipFree(c->mom);
@@ -466,9 +466,8 @@ long yh_volume(const yh_ctx* c) { return c ? c->g.V : -1; }
 int yh_set_gauge(yh_ctx* c, const double* links) {
   if (!c || !links) { set_error("null argument"); return YH_ERR_ARG; }
   YH_HIP(hipSetDevice(c->device));
-  size_t n = (size_t)4 * c->g.V * 2 * c->nc * c->nc;
-  YH_HIP(hipMemcpyAsync(c->fund, links, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
   int rc;
+  if ((rc = gauge_upload(c, links))) return rc;
   if ((rc = gauge_represent(c))) return rc;
   if ((rc = gauge_derive_links(c))) return rc;
   if ((rc = clover_build(c))) return rc;

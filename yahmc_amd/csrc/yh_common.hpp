@@ -152,6 +152,26 @@ __device__ __forceinline__ double bc_cf_shift(int t, const Geom& g) {
   return 0.0;
 }
 
+// coordinates of c + d e_dir (d between -L and L, periodic wrap) and their
+// full-lattice EO index; dir may be a run-time value
+__device__ __forceinline__ int neighbour(const int (&c)[4], int dir, int d, const Geom& g, int (&o)[4]) {
+#pragma unroll
+  for (int a = 0; a < 4; a++) {
+    int v = c[a] + (a == dir ? d : 0);
+    v = v < 0 ? v + g.L[a] : (v >= g.L[a] ? v - g.L[a] : v);
+    o[a] = v;
+  }
+  return full_index(o[0], o[1], o[2], o[3], g);
+}
+
+// element 0 of the fundamental link (id, mu) in the component-plane layout
+// (the layout of the represented links); its elements are VHpad apart
+template <int NC>
+__device__ __forceinline__ size_t fund_at(int id, int mu, const Geom& g) {
+  const int p = id >= g.VH;
+  return (size_t)(p * 4 + mu) * NC * NC * g.VHpad + (id - p * g.VH);
+}
+
 // XCD-aware block order.  The hardware deals consecutive workgroups round
 // robin to the 8 XCDs (physical block b runs on XCD b % 8 as that XCD's
 // (b / 8)-th block).  Remap so that XCD x takes `q` consecutive logical

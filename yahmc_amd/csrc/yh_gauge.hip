@@ -74,12 +74,13 @@ int gauge_init_basis(Ctx* c) {
 typedef Cx<double> cd;
 
 template <int NC>
-__device__ __forceinline__ void load_fund(cd (&u)[NC][NC], const double* fund, int id, int mu) {
-  const double* p = fund + (size_t)(4 * id + mu) * 2 * NC * NC;
+__device__ __forceinline__ void load_fund(cd (&u)[NC][NC], const double2* fund, int id, int mu, const Geom& g) {
+  const double2* p = fund + fund_at<NC>(id, mu, g);
 #pragma unroll
-  for (int i = 0; i < NC; i++)
-#pragma unroll
-    for (int j = 0; j < NC; j++) u[i][j] = cd(p[i * NC + j], p[NC * NC + i * NC + j]);
+  for (int e = 0; e < NC * NC; e++) {
+    const double2 v = p[(size_t)e * g.VHpad];
+    u[e / NC][e % NC] = cd(v.x, v.y);
+  }
 }
 
 template <int NC>
@@ -177,15 +178,14 @@ __device__ __forceinline__ void represent(cd (&R)[D][D], const cd (&U)[NC][NC], 
   }
 }
 
-// fund links (reference AoS) -> F64 recon-18 SoA links (no BC sign)
+// fundamental links -> F64 recon-18 represented links (no BC sign)
 template <int NC, int REPR, int D>
-__global__ void k_represent(const double* __restrict__ fund, double2* __restrict__ out, Geom g,
+__global__ void k_represent(const double2* __restrict__ fund, double2* __restrict__ out, Geom g,
                             const double2* __restrict__ basis) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 4 * g.V) return;
-  int id = t >> 2, mu = t & 3;
+  const int id = blockIdx.x * blockDim.x + threadIdx.x, mu = blockIdx.y;
+  if (id >= g.V) return;
   cd U[NC][NC], R[D][D];
-  load_fund<NC>(U, fund, id, mu);
+  load_fund<NC>(U, fund, id, mu, g);
   represent<NC, REPR, D>(R, U, basis);
   int p = id >= g.VH;
   int k = id - p * g.VH;
@@ -262,7 +262,7 @@ __device__ __forceinline__ void load_packed(cd (&M)[N][N], const double2* base, 
 __device__ __forceinline__ void cb_fence() { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront"); }
 
 template <int NC, int REPR, int D>
-__global__ void __launch_bounds__(64) k_clover_build_rows(const double* __restrict__ fund, double2* __restrict__ out,
+__global__ void __launch_bounds__(64) k_clover_build_rows(const double2* __restrict__ fund, double2* __restrict__ out,
                                                          Geom g, double csw, const double2* __restrict__ basis) {
   constexpr int G = 64 / D, N = 2 * D, NN = NC * NC;
   __shared__ double2 lv[G][4][NN];  // the plane's four leaves
@@ -329,13 +329,13 @@ __global__ void __launch_bounds__(64) k_clover_build_rows(const double* __restri
       // place row by row
       cd L[NC][NC], F[NC][NC];
       auto ldf = [&](cd (&u)[NC][NC], int st, int dr, bool dg) {
-        const double* pf = fund + (size_t)(4 * st + dr) * 2 * NC * NC;
+        const double2* pf = fund + fund_at<NC>(st, dr, g);
 #pragma unroll
         for (int a = 0; a < NC; a++)
 #pragma unroll
           for (int b = 0; b < NC; b++) {
-            const int e = dg ? b * NC + a : a * NC + b;
-            u[a][b] = cd(pf[e], dg ? -pf[NC * NC + e] : pf[NC * NC + e]);
+            const double2 v = pf[(size_t)(dg ? b * NC + a : a * NC + b) * g.VHpad];
+            u[a][b] = cd(v.x, dg ? -v.y : v.y);
           }
       };
       ldf(L, s[0], d[0], h[0]);
@@ -675,7 +675,7 @@ int gauge_represent(Ctx* c) {
     YH_HIP(hipMalloc(&c->links[PREC_F64][RECON_18], bytes));
   }
   double2* out = (double2*)c->links[PREC_F64][RECON_18];
-  YH_ALL_MODELS(hipLaunchKernelGGL((k_represent<NC_, REPR_, D_>), dim3(grid1(4L * c->g.V)), dim3(256), 0, c->stream,
+  YH_ALL_MODELS(hipLaunchKernelGGL((k_represent<NC_, REPR_, D_>), dim3(grid1(c->g.V), 4), dim3(256), 0, c->stream,
                                    c->fund, out, c->g, c->tab_basis);
                 YH_HIP(hipGetLastError()));
   set_error("unsupported (nc, repr) model");

@@ -60,8 +60,11 @@ struct Ctx {
   int device;
   hipStream_t stream;
   int nblk;            // blocks of 256 threads over one half
-  // gauge field: fundamental links in the reference layout (4V suNg)
-  double* fund = nullptr;
+  // gauge field: fundamental links, component planes like the represented
+  // links (yh_common.hpp), and the buffer that host transfers in the
+  // reference layout (4V suNg) go through
+  double2* fund = nullptr;
+  double* fund_aos = nullptr;
   // represented links, SoA, per (prec, recon); null if not built
   void* links[3][2] = {{nullptr, nullptr}, {nullptr, nullptr}, {nullptr, nullptr}};
   // packed clover term (no mass) for both parities, per precision
@@ -106,12 +109,11 @@ struct Ctx {
   int use_graphs = 1;
   // model tables of this context's (nc, representation), in device memory
   // and passed to the kernels as arguments (two live contexts of different
-  // models each keep their own): representation basis b_n, represented
-  // generators iT^R_a and fundamental generators iT_a
+  // models each keep their own): representation basis b_n and represented
+  // generators iT^R_a
   double2* tab = nullptr;
   double2* tab_basis = nullptr;  // TAB_BASIS entries
   double2* tab_itr = nullptr;    // TAB_ITR entries
-  double2* tab_itf = nullptr;    // TAB_ITF entries
   // pinned host copy of the last reduction read back (2 doubles)
   double* red_host = nullptr;
   // caller-provided temporaries (the no-allocation entry point): when set,
@@ -120,7 +122,7 @@ struct Ctx {
   Field* op_tmp[2] = {nullptr, nullptr};
   Field* cg_tmp[3] = {nullptr, nullptr, nullptr};
 };
-enum { TAB_BASIS = 15 * 16, TAB_ITR = 15 * 64, TAB_ITF = 15 * 16 };
+enum { TAB_BASIS = 15 * 16, TAB_ITR = 15 * 64 };
 // copies `n` table entries to device memory on the context stream and waits
 int upload_table(Ctx* c, double2* dst, const double2* host, size_t n);
 
@@ -135,6 +137,8 @@ int field_convert(Ctx* c, Field* dst, int dpar, const Field* src, int spar);
 
 // ---- gauge ------------------------------------------------------------------
 int gauge_init_basis(Ctx* c);
+int gauge_upload(Ctx* c, const double* host);    // host links (4V suNg) -> fund
+int gauge_download(Ctx* c, double* host);        // fund -> host links
 int gauge_represent(Ctx* c);                 // fund -> F64 R18 links
 int gauge_derive_links(Ctx* c);              // F64 R18 -> other precisions
 int clover_build(Ctx* c);                    // packed FP64 clover
@@ -193,7 +197,6 @@ int momenta_download(Ctx* c, double* host);
 int clover_force_download(Ctx* c, double* host);
 
 // ---- gauge molecular dynamics ----------------------------------------------
-int md_init_constants(Ctx* c);
 int md_gauge_force(Ctx* c, double dt, double beta);
 int md_improved_gauge_force(Ctx* c, double dt, double beta, double c0, double c1);
 int md_avr_wilson(Ctx* c, int h, int w, double* out);

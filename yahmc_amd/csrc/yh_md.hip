@@ -9,11 +9,13 @@
 // avr_wilson(h, w)   : library/wilsonloop.cpp:58-133 (rectangle weights of
 //                      bcs.cpp:30-31, 72-120)
 // hamiltonian (P^2)  : library/update.cpp:201-216
-// Fundamental links stay in the reference layout (4*id+mu, re plane then im
-// plane); momenta are SoA mom[(mu * NG + a) * V + id].  Periodic, open and
+// Fundamental links are kept as component planes (the layout of the
+// represented links): a wave of 64 consecutive sites of one parity and one
+// direction reads each element as one contiguous 1 KB segment.  Host
+// transfers in the reference layout (4*id+mu, re plane then im plane) are
+// transposed through LDS.  Momenta are SoA mom[(mu * NG + a) * V + id].  Periodic, open and
 // SF gauge boundaries (bcs.cpp: boundary plaquette weights, fixed links).
 #include <algorithm>
-#include <vector>
 #include "yh_internal.hpp"
 #include "yh_reduce.hpp"
 
@@ -32,26 +34,75 @@ struct M {
 };
 
 template <int NC>
-__device__ __forceinline__ M<NC> ld(const double* fund, int id, int mu) {
+__device__ __forceinline__ M<NC> ld(const double2* fund, int id, int mu, const Geom& g) {
   M<NC> u;
-  const double* p = fund + (size_t)(4 * id + mu) * 2 * NC * NC;
+  const double2* p = fund + fund_at<NC>(id, mu, g);
 #pragma unroll
-  for (int i = 0; i < NC; i++)
+  for (int e = 0; e < NC * NC; e++) {
+    const double2 v = p[(size_t)e * g.VHpad];
+    u.m[e / NC][e % NC] = cd(v.x, v.y);
+  }
+  return u;
+}
+
+// conjugate transpose of the link
+template <int NC>
+__device__ __forceinline__ M<NC> ldd(const double2* fund, int id, int mu, const Geom& g) {
+  M<NC> u;
+  const double2* p = fund + fund_at<NC>(id, mu, g);
 #pragma unroll
-    for (int j = 0; j < NC; j++) u.m[i][j] = cd(p[i * NC + j], p[NC * NC + i * NC + j]);
+  for (int e = 0; e < NC * NC; e++) {
+    const double2 v = p[(size_t)e * g.VHpad];
+    u.m[e % NC][e / NC] = cd(v.x, -v.y);
+  }
   return u;
 }
 
 template <int NC>
-__device__ __forceinline__ void st(double* fund, int id, int mu, const M<NC>& u) {
-  double* p = fund + (size_t)(4 * id + mu) * 2 * NC * NC;
+__device__ __forceinline__ void st(double2* fund, int id, int mu, const M<NC>& u, const Geom& g) {
+  double2* p = fund + fund_at<NC>(id, mu, g);
 #pragma unroll
-  for (int i = 0; i < NC; i++)
-#pragma unroll
-    for (int j = 0; j < NC; j++) {
-      p[i * NC + j] = u.m[i][j].re;
-      p[NC * NC + i * NC + j] = u.m[i][j].im;
+  for (int e = 0; e < NC * NC; e++)
+    p[(size_t)e * g.VHpad] = make_double2(u.m[e / NC][e % NC].re, u.m[e / NC][e % NC].im);
+}
+
+// host layout <-> component planes: a block moves AS sites of one parity
+// (contiguous in both layouts) through LDS, so that both sides are coalesced
+template <int NC>
+struct AosTile {
+  static constexpr int S = NC == 4 ? 32 : 64;   // sites
+  static constexpr int W = 8 * NC * NC;          // doubles of a site's four links
+};
+
+template <int NC, bool TO_AOS>
+__global__ void __launch_bounds__(256) k_fund_aos(double* __restrict__ aos, double2* __restrict__ fund, Geom g) {
+  typedef AosTile<NC> A;
+  constexpr int NN = NC * NC;
+  __shared__ double tile[A::S * (A::W + 1)];  // the odd site stride spreads the banks
+  const int p = blockIdx.y, k0 = blockIdx.x * A::S;
+  const int n = min(A::S, g.VH - k0);
+  double* base = aos + (size_t)(p * g.VH + k0) * A::W;
+  if (!TO_AOS) {
+    for (int i = threadIdx.x; i < n * A::W; i += 256) tile[(i / A::W) * (A::W + 1) + i % A::W] = base[i];
+    __syncthreads();
+  }
+  for (int j = threadIdx.x; j < 4 * NN * A::S; j += 256) {
+    const int s = j % A::S, mu = j / A::S / NN, e = j / A::S % NN;
+    if (s >= n) continue;
+    double2* f = fund + ((size_t)(p * 4 + mu) * NN + e) * g.VHpad + k0 + s;
+    double* t = tile + s * (A::W + 1) + mu * 2 * NN + e;
+    if (TO_AOS) {
+      const double2 v = *f;
+      t[0] = v.x;
+      t[NN] = v.y;
+    } else {
+      *f = make_double2(t[0], t[NN]);
     }
+  }
+  if (TO_AOS) {
+    __syncthreads();
+    for (int i = threadIdx.x; i < n * A::W; i += 256) base[i] = tile[(i / A::W) * (A::W + 1) + i % A::W];
+  }
 }
 
 template <int NC>
@@ -99,12 +150,6 @@ __device__ __forceinline__ M<NC> dmul(const M<NC>& a, const M<NC>& b) {
       r.m[i][j] = s;
     }
   return r;
-}
-
-__device__ __forceinline__ int mshift(const int c[4], int mu, int d, const Geom& g) {
-  int n[4] = {c[0], c[1], c[2], c[3]};
-  n[mu] = (n[mu] + d + g.L[mu]) % g.L[mu];
-  return full_index(n[0], n[1], n[2], n[3], g);
 }
 
 // anti-Hermitian matrix of an algebra vector (library/suNg.cpp:15-58)
@@ -247,9 +292,6 @@ __device__ __forceinline__ void reunit(M<NC>& u) {
   }
 }
 
-// fundamental generators iT_a, NC x NC: the context's table
-// tab_itf[a * 16 + i * NC + k], passed to the kernels
-
 // Open and SF boundaries of the gauge field (library/bcs.cpp:28-130, 166-262):
 // spatial plaquettes based on the boundary slices (open: t = 0 and T-1; SF:
 // t = 0 and T-2) count half in the action and its force, and the links the
@@ -285,13 +327,13 @@ __device__ __forceinline__ double rect_w(int t, int a, int b, const Geom& g) {
 // U(c, d) and moves to c + d; backward (d, -1) moves to c - d and multiplies
 // by U(c - d, d)^+
 template <int NC>
-__device__ __forceinline__ void path_step(M<NC>& P, const double* fund, int (&c)[4], int d, bool fw, const Geom& g) {
+__device__ __forceinline__ void path_step(M<NC>& P, const double2* fund, int (&c)[4], int d, bool fw, const Geom& g) {
   if (fw) {
-    P = mul<NC>(P, ld<NC>(fund, full_index(c[0], c[1], c[2], c[3], g), d));
+    P = mul<NC>(P, ld<NC>(fund, full_index(c[0], c[1], c[2], c[3], g), d, g));
     c[d] = c[d] + 1 == g.L[d] ? 0 : c[d] + 1;
   } else {
     c[d] = c[d] == 0 ? g.L[d] - 1 : c[d] - 1;
-    P = muld<NC>(P, ld<NC>(fund, full_index(c[0], c[1], c[2], c[3], g), d));
+    P = muld<NC>(P, ld<NC>(fund, full_index(c[0], c[1], c[2], c[3], g), d, g));
   }
 }
 
@@ -304,23 +346,6 @@ __device__ __forceinline__ M<NC> unit_matrix() {
     for (int j = 0; j < NC; j++) r.m[i][j] = cd(i == j ? 1.0 : 0.0, 0.0);
   return r;
 }
-
-// The six 1 x 2 rectangles through the link (x, mu) for one nu, as paths
-// from x + mu back to x (bits 2j, 2j+1 of the code: step j is 0 +mu, 1 -mu,
-// 2 +nu, 3 -nu), with the offset of the rectangle's base corner from x
-// (bits 10-11: -mu steps, 12-13: -nu steps) and whether its long side is
-// along nu (bit 14), which orders the arguments of its weight
-#define YH_R(s0, s1, s2, s3, s4, bm, bn, lnu) \
-  ((s0) | (s1) << 2 | (s2) << 4 | (s3) << 6 | (s4) << 8 | (bm) << 10 | (bn) << 12 | (lnu) << 14)
-__constant__ int c_rect_paths[6] = {
-    YH_R(2, 2, 1, 3, 3, 0, 0, 1),  // long side nu, +nu side
-    YH_R(3, 3, 1, 2, 2, 0, 2, 1),  // long side nu, -nu side
-    YH_R(0, 2, 1, 1, 3, 0, 0, 0),  // long side mu, the link first, +nu side
-    YH_R(2, 1, 1, 3, 0, 1, 0, 0),  // long side mu, the link second, +nu side
-    YH_R(0, 3, 1, 1, 2, 0, 1, 0),  // long side mu, the link first, -nu side
-    YH_R(3, 1, 1, 2, 0, 1, 1, 0),  // long side mu, the link second, -nu side
-};
-#undef YH_R
 
 // apply_bcs_on_momentum_field (bcs.cpp:166-199)
 __global__ void __launch_bounds__(256) k_mom_bcs(double* __restrict__ mom, int NG, Geom g) {
@@ -336,10 +361,9 @@ __global__ void __launch_bounds__(256) k_mom_bcs(double* __restrict__ mom, int N
 // apply_bcs_on_gauge_field (bcs.cpp:201-262): the fixed links take their
 // boundary values: zero, or the SF matrices diag(exp(i c1_k)), diag(exp(i c2_k))
 template <int NC>
-__global__ void __launch_bounds__(256) k_gauge_bcs(double* __restrict__ fund, Geom g, SfPhases ph) {
-  int t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= 4 * g.V) return;
-  int id = t >> 2, mu = t & 3;
+__global__ void __launch_bounds__(256) k_gauge_bcs(double2* __restrict__ fund, Geom g, SfPhases ph) {
+  const int id = blockIdx.x * 256 + threadIdx.x, mu = blockIdx.y;
+  if (id >= g.V) return;
   int c[4];
   full_coords(id, g, c);
   if (!link_fixed(c[0], mu, g)) return;
@@ -353,92 +377,231 @@ __global__ void __launch_bounds__(256) k_gauge_bcs(double* __restrict__ fund, Ge
 #pragma unroll
     for (int i = 0; i < NC; i++) u.m[i][i] = cd(cos(v[i]), sin(v[i]));
   }
-  st<NC>(fund, id, mu, u);
+  st<NC>(fund, id, mu, u, g);
 }
 
-// Wilson gauge force: mom -= algebra_project(U staple, dt beta / NC), the
-// staples weighted by their plaquettes' weights (staples.cpp:82-107).  With
-// RECT the improved force: staple c0 S_plaq + c1 S_rect, S_rect the six
-// weighted rectangles through the link for each nu (staples.cpp:7-80)
-template <int NC, bool RECT>
-__global__ void __launch_bounds__(128) k_gauge_force(const double* __restrict__ fund, double* __restrict__ mom,
-                                                     double coeff, double c0, double c1, Geom g,
-                                                     const double2* __restrict__ itf) {
-  int t = blockIdx.x * 128 + threadIdx.x;
-  if (t >= 4 * g.V) return;
-  int id = t >> 2, mu = t & 3;
-  constexpr int NG = NC * NC - 1;
-  int c[4];
-  full_coords(id, g, c);
-  M<NC> S;
+template <int NC>
+__device__ __forceinline__ void axpy(M<NC>& s, double w, const M<NC>& a) {
 #pragma unroll
   for (int i = 0; i < NC; i++)
 #pragma unroll
-    for (int j = 0; j < NC; j++) S.m[i][j] = cd(0, 0);
-  int o1m = mshift(c, mu, 1, g);
-  for (int nu = 0; nu < 4; nu++) {
-    if (nu == mu) continue;
-    int o2 = mshift(c, nu, 1, g);
-    M<NC> a = mul<NC>(ld<NC>(fund, id, nu), ld<NC>(fund, o2, mu));
-    M<NC> s1 = muld<NC>(ld<NC>(fund, o1m, nu), a);
-    int b = mshift(c, nu, -1, g);
-    int cb[4];
-    full_coords(b, g, cb);
-    int b2 = mshift(cb, mu, 1, g);
-    M<NC> q = mul<NC>(ld<NC>(fund, b, mu), ld<NC>(fund, b2, nu));
-    M<NC> s2 = dmul<NC>(q, ld<NC>(fund, b, nu));
-    double w1 = plaq_w(c[0], mu, nu, g), w2 = plaq_w(cb[0], nu, mu, g);
-    if constexpr (RECT) {
-      w1 *= c0;
-      w2 *= c0;
+    for (int j = 0; j < NC; j++) {
+      s.m[i][j].re = fma(w, a.m[i][j].re, s.m[i][j].re);
+      s.m[i][j].im = fma(w, a.m[i][j].im, s.m[i][j].im);
     }
+}
+
+template <int NC>
+__device__ __forceinline__ M<NC> scaled(double w, const M<NC>& a) {
+  M<NC> r;
 #pragma unroll
-    for (int i = 0; i < NC; i++)
+  for (int i = 0; i < NC; i++)
 #pragma unroll
-      for (int j = 0; j < NC; j++) S.m[i][j] = S.m[i][j] + w1 * s1.m[i][j] + w2 * s2.m[i][j];
-    if constexpr (RECT) {
-      for (int r = 0; r < 6; r++) {
-        const int code = c_rect_paths[r];
-        int p[4] = {c[0], c[1], c[2], c[3]};
-        p[mu] = p[mu] + 1 == g.L[mu] ? 0 : p[mu] + 1;
-        M<NC> P = unit_matrix<NC>();
-        for (int j = 0; j < 5; j++) {
-          const int sc = (code >> (2 * j)) & 3;
-          path_step<NC>(P, fund, p, sc >> 1 ? nu : mu, (sc & 1) == 0, g);
-        }
-        // time slice of the base corner: x - bm mu - bn nu
-        int tb = c[0] - (mu == 0 ? (code >> 10) & 3 : 0) - (nu == 0 ? (code >> 12) & 3 : 0);
-        tb = tb < 0 ? tb + g.L[0] : tb;
-        const double w = c1 * ((code >> 14) & 1 ? rect_w(tb, mu, nu, g) : rect_w(tb, nu, mu, g));
+    for (int j = 0; j < NC; j++) r.m[i][j] = w * a.m[i][j];
+  return r;
+}
+
+// an opaque zero once every element of m is final: link indices that it is
+// added to are loaded after m, so that the loads of a chain of products are
+// not all issued (and held in registers) at its start
+template <int NC>
+__device__ __forceinline__ int settled(M<NC>& m) {
 #pragma unroll
-        for (int i = 0; i < NC; i++)
+  for (int i = 0; i < NC; i++)
 #pragma unroll
-          for (int j = 0; j < NC; j++) S.m[i][j] = S.m[i][j] + w * P.m[i][j];
+    for (int j = 0; j < NC; j++) __asm__ volatile("" : "+v"(m.m[i][j].re), "+v"(m.m[i][j].im));
+  int z;
+  __asm__ volatile("v_mov_b32 %0, 0" : "=v"(z));
+  return z;
+}
+
+// Re Tr(iT_a F) of every generator, in the reference's order
+// (suNa.cpp:102-111): each has two entries, or the i + 1 of a diagonal one
+template <int NC>
+__device__ __forceinline__ void project(double (&out)[NC * NC - 1], const M<NC>& F) {
+  int a = 0;
+#pragma unroll
+  for (int i = 0; i < NC; i++)
+#pragma unroll
+    for (int j = 0; j < NC; j++) {
+      if (i > j) {
+        out[a++] = -F.m[j][i].im - F.m[i][j].im;
+      } else if (i < j) {
+        out[a++] = F.m[j][i].re - F.m[i][j].re;
+      } else if (i > 0) {
+        double re = i * F.m[i][i].im;
+#pragma unroll
+        for (int k = 0; k < i; k++) re -= F.m[k][k].im;
+        out[a++] = re * sqrt(2.0 / (i * (i + 1)));
       }
     }
+}
+
+// Work order of the gauge-force kernels: mu fastest, then parity, then blocks
+// of 64 sites, so that the workgroups that share links run side by side; each
+// XCD takes 64 consecutive workgroups in turn, which keeps the time
+// neighbours of its sites closer than one contiguous slab per XCD does
+// (SU(3) Wilson force at 32^4: 690 us, one slab per XCD 746).
+struct ForceItem {
+  int mu, p, k;  // direction, parity, half index (may lie past the end)
+};
+__device__ __forceinline__ ForceItem force_item() {
+  const int b = xcd_block(gridDim.x, 64);
+  return ForceItem{b & 3, (b >> 2) & 1, (b >> 3) * 64 + (int)(threadIdx.x & 63)};
+}
+
+// The tail of a gauge-force workgroup: the waves' staples S meet in LDS and
+// are added in a fixed order, and wave 0 projects U(x, mu) S onto the momenta.
+template <int NC, int NW>
+__device__ __forceinline__ void force_tail(M<NC>& S, const double2* fund, double* mom, double f, int w, int lane,
+                                           const ForceItem& it, const Geom& g) {
+  constexpr int NN = NC * NC, NG = NN - 1;
+  __shared__ double2 ex[NW - 1][NN][64];
+  if (w > 0) {
+#pragma unroll
+    for (int e = 0; e < NN; e++) ex[w - 1][e][lane] = make_double2(S.m[e / NC][e % NC].re, S.m[e / NC][e % NC].im);
   }
-  M<NC> F = mul<NC>(ld<NC>(fund, id, mu), S);
+  __syncthreads();
+  if (w > 0 || it.k >= g.VH) return;
 #pragma unroll
-  for (int a = 0; a < NG; a++) {
-    double re = 0;
+  for (int q = 0; q < NW - 1; q++)
 #pragma unroll
-    for (int i = 0; i < NC; i++)
+    for (int e = 0; e < NN; e++) {
+      const double2 v = ex[q][e][lane];
+      S.m[e / NC][e % NC] = S.m[e / NC][e % NC] + cd(v.x, v.y);
+    }
+  const int id = it.p * g.VH + it.k;
+  double a[NG];
+  project<NC>(a, mul<NC>(ld<NC>(fund, id, it.mu, g), S));
 #pragma unroll
-      for (int k = 0; k < NC; k++) {
-        double2 tg = itf[a * 16 + i * NC + k];
-        re += tg.x * F.m[k][i].re - tg.y * F.m[k][i].im;
-      }
-    mom[(size_t)(mu * NG + a) * g.V + id] -= -(coeff * 0.5) * re;
+  for (int n = 0; n < NG; n++) mom[(size_t)(it.mu * NG + n) * g.V + id] += f * a[n];
+}
+
+// Wilson gauge force: mom -= algebra_project(U staple, dt beta / NC), the
+// staples weighted by their plaquettes' weights (forces.cpp:262-283,
+// staples.cpp:82-107).  A workgroup takes 64 consecutive sites of one parity
+// and one mu, one wave per nu.  Bound by the 19 link reads per (x, mu) from
+// L2: 690 us at 32^4 (16.6 TB/s of link reads; 1,614 us with the links as an
+// array of 144-byte structures, where every load of a wave touches 64 or
+// more cache lines, and one thread per link).  Measured and not kept: one
+// wave per plane forming the plaquettes that serve two links each (fewer
+// reads, but 217 registers and two waves per SIMD: 923 us), and one wave per
+// (nu, side) (1,015 us).
+template <int NC>
+__global__ void __launch_bounds__(192) k_wilson_force(const double2* __restrict__ fund, double* __restrict__ mom,
+                                                      double f, Geom g) {
+  const ForceItem it = force_item();
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kk = min(it.k, g.VH - 1);  // lanes past the end compute on the last site and write nothing
+  const int id = it.p * g.VH + kk, mu = it.mu, nu = w + (w >= mu);
+  int c[4], cb[4], q[4];
+  site_coords(kk, it.p, g, c);
+  const int om = neighbour(c, mu, 1, g, q), on = neighbour(c, nu, 1, g, q);
+  const int bn = neighbour(c, nu, -1, g, cb), bnm = neighbour(cb, mu, 1, g, q);
+  auto L = [&](int i, int d) { return ld<NC>(fund, i, d, g); };
+  M<NC> S = scaled(plaq_w(c[0], mu, nu, g), muld(L(om, nu), mul(L(id, nu), L(on, mu))));
+  axpy(S, plaq_w(cb[0], nu, mu, g), dmul(mul(L(bn, mu), L(bnm, nu)), L(bn, nu)));
+  force_tail<NC, 3>(S, fund, mom, f, w, lane, it, g);
+}
+
+// the weighted staples of the link (x, mu) on one side (UP: +nu) of it,
+// paths from x + mu back to x.  With A = U(x+mu, nu), B = U(x+nu, mu)^+,
+// C = U(x, nu)^+ (down: the links around the plaquette at x - nu) the
+// plaquette staple is A B C, and each of the three 1 x 2 rectangles on this
+// side replaces one of the three links by its own staple: A P C (long side
+// along nu), Q B C and A B R (long side along mu).  Summed as
+//   A (w0 B C + wP P C + wR B R) + wQ Q (B C):
+// 11 products, against 17 for the four paths taken one by one.
+template <int NC, bool UP>
+__device__ __forceinline__ M<NC> side_staple(const double2* fund, const int (&c)[4], int id, int mu, int nu, double c0,
+                                             double c1, const Geom& g) {
+  auto L = [&](int i, int d) { return ld<NC>(fund, i, d, g); };
+  auto D = [&](int i, int d) { return ldd<NC>(fund, i, d, g); };
+  int cn[4], cm[4], cmn[4], q[4], r[4];
+  const int om = neighbour(c, mu, 1, g, cm);
+  const int on = neighbour(c, nu, UP ? 1 : -1, g, cn);    // x +- nu
+  const int omn = neighbour(cn, mu, 1, g, cmn);           // x + mu +- nu
+  const int dt = nu == 0 ? (UP ? 0 : -1) : 0;             // time of the base corner of the plaquette, less t
+  auto wrap = [&](int t) { return t < 0 ? t + g.L[0] : t; };
+  const double w0 = plaq_w(wrap(c[0] + dt), mu, nu, g);
+  const double wP = c1 * rect_w(wrap(c[0] + 2 * dt), mu, nu, g);
+  const double wQ = c1 * rect_w(wrap(c[0] + dt), nu, mu, g);
+  const double wR = c1 * rect_w(wrap(c[0] + dt - (mu == 0)), nu, mu, g);
+  const M<NC> B = D(on, mu);
+  const M<NC> C = UP ? D(id, nu) : L(on, nu);
+  const M<NC> BC = mul(B, C);
+  M<NC> T = scaled(w0 * c0, BC);
+  {
+    // P: the staple of (x +- nu, mu) one step further along nu
+    const int z = settled(T);
+    const int o2n = neighbour(cn, nu, UP ? 1 : -1, g, q) + z;   // x +- 2 nu
+    const int om2n = neighbour(q, mu, 1, g, r) + z;             // x + mu +- 2 nu
+    M<NC> P = UP ? muld(L(omn + z, nu), L(o2n, mu)) : mul(D(om2n, nu), D(o2n, mu));
+    P = UP ? muld(P, L(on + z, nu)) : mul(P, L(o2n, nu));
+    axpy(T, wP, mul(P, C));
   }
+  {
+    // R: around the plaquette at x - mu (+- nu)
+    const int z = settled(T);
+    const int ob = neighbour(c, mu, -1, g, q) + z;              // x - mu
+    const int obn = neighbour(cn, mu, -1, g, r) + z;            // x - mu +- nu
+    M<NC> R = mul(D(obn, mu), UP ? D(ob, nu) : L(obn, nu));
+    R = mul(R, L(ob, mu));
+    axpy(T, wR, mul(B, R));
+  }
+  const int z = settled(T);
+  M<NC> S = mul(UP ? L(om + z, nu) : D(omn + z, nu), T);
+  {
+    // Q: around the plaquette at x + mu (+- nu)
+    const int z2 = settled(S);
+    const int o2m = neighbour(cm, mu, 1, g, q) + z2;            // x + 2 mu
+    const int o2mn = neighbour(cmn, mu, 1, g, r) + z2;          // x + 2 mu +- nu
+    M<NC> Q = UP ? mul(L(om + z2, mu), L(o2m, nu)) : muld(L(om + z2, mu), L(o2mn, nu));
+    Q = muld(Q, L(omn + z2, mu));
+    axpy(S, wQ, mul(Q, BC));
+  }
+  return S;
+}
+
+// Improved gauge force: mom -= algebra_project(U staple, dt beta / NC) with
+// staple = c0 S_plaq + c1 S_rect, S_rect the six weighted rectangles through
+// the link for each nu (forces.cpp:285-310, staples.cpp:7-80).
+// A workgroup takes 64 consecutive sites of one parity and one mu; its waves
+// share out the six (nu, side), add their staples through LDS in a fixed
+// order, and wave 0 multiplies by the link and projects.
+// waves of a workgroup (SU(4) keeps both sides in a wave: the exchange of six takes 80 KB of LDS)
+constexpr int rect_waves(int nc) { return nc < 4 ? 6 : 3; }
+
+template <int NC>
+__global__ void __launch_bounds__((64 * rect_waves(NC))) k_rect_force(const double2* __restrict__ fund,
+                                                                     double* __restrict__ mom, double f, double c0,
+                                                                     double c1, Geom g) {
+  constexpr int NW = rect_waves(NC);
+  const ForceItem it = force_item();
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kk = min(it.k, g.VH - 1);  // lanes past the end compute on the last site and write nothing
+  const int id = it.p * g.VH + kk, mu = it.mu;
+  int c[4];
+  site_coords(kk, it.p, g, c);
+  const int j = NW == 6 ? w >> 1 : w;
+  const int nu = j + (j >= mu);
+  M<NC> S;
+  if constexpr (NW == 6) {
+    if (w & 1) S = side_staple<NC, false>(fund, c, id, mu, nu, c0, c1, g);
+    else S = side_staple<NC, true>(fund, c, id, mu, nu, c0, c1, g);
+  } else {
+    S = side_staple<NC, true>(fund, c, id, mu, nu, c0, c1, g);
+    axpy(S, 1.0, side_staple<NC, false>(fund, c, id + settled(S), mu, nu, c0, c1, g));
+  }
+  force_tail<NC, NW>(S, fund, mom, f, w, lane, it, g);
 }
 
 // U <- exp(eps P) U, Taylor series to |X^k/k!|^2 < 1e-24 then reunitarised
 template <int NC>
-__global__ void __launch_bounds__(128) k_update_links(double* __restrict__ fund, const double* __restrict__ mom,
+__global__ void __launch_bounds__(128) k_update_links(double2* __restrict__ fund, const double* __restrict__ mom,
                                                       double eps, Geom g) {
-  int t = blockIdx.x * 128 + threadIdx.x;
-  if (t >= 4 * g.V) return;
-  int id = t >> 2, mu = t & 3;
+  const int id = blockIdx.x * 128 + threadIdx.x, mu = blockIdx.y;
+  if (id >= g.V) return;
   M<NC> X = alg<NC>(mom, g.V, mu, id);
   M<NC> R, Xk;
 #pragma unroll
@@ -463,21 +626,21 @@ __global__ void __launch_bounds__(128) k_update_links(double* __restrict__ fund,
       }
   }
   reunit<NC>(R);
-  st<NC>(fund, id, mu, mul<NC>(R, ld<NC>(fund, id, mu)));
+  st<NC>(fund, id, mu, mul<NC>(R, ld<NC>(fund, id, mu, g)), g);
 }
 
 template <int NC>
-__global__ void __launch_bounds__(128) k_reunitarize(double* __restrict__ fund, Geom g) {
-  int t = blockIdx.x * 128 + threadIdx.x;
-  if (t >= 4 * g.V) return;
-  M<NC> u = ld<NC>(fund, t >> 2, t & 3);
+__global__ void __launch_bounds__(128) k_reunitarize(double2* __restrict__ fund, Geom g) {
+  const int id = blockIdx.x * 128 + threadIdx.x, mu = blockIdx.y;
+  if (id >= g.V) return;
+  M<NC> u = ld<NC>(fund, id, mu, g);
   reunit<NC>(u);
-  st<NC>(fund, t >> 2, t & 3, u);
+  st<NC>(fund, id, mu, u, g);
 }
 
 // sum over planes of Re Tr of the plaquette
 template <int NC>
-__global__ void __launch_bounds__(256) k_plaquette(const double* __restrict__ fund, double* partials, unsigned* ticket,
+__global__ void __launch_bounds__(256) k_plaquette(const double2* __restrict__ fund, double* partials, unsigned* ticket,
                                                    double* out, Geom g) {
   int id = blockIdx.x * 256 + threadIdx.x;
   double v[1] = {0.0};
@@ -486,9 +649,10 @@ __global__ void __launch_bounds__(256) k_plaquette(const double* __restrict__ fu
     full_coords(id, g, c);
     for (int mu = 1; mu < 4; mu++)
       for (int nu = 0; nu < mu; nu++) {
-        int a = mshift(c, mu, 1, g), b = mshift(c, nu, 1, g);
-        M<NC> one = mul<NC>(ld<NC>(fund, id, mu), ld<NC>(fund, a, nu));
-        M<NC> two = mul<NC>(ld<NC>(fund, id, nu), ld<NC>(fund, b, mu));
+        int o[4];
+        const int a = neighbour(c, mu, 1, g, o), b = neighbour(c, nu, 1, g, o);
+        M<NC> one = mul<NC>(ld<NC>(fund, id, mu, g), ld<NC>(fund, a, nu, g));
+        M<NC> two = mul<NC>(ld<NC>(fund, id, nu, g), ld<NC>(fund, b, mu, g));
         M<NC> P = muld<NC>(one, two);
         double tr = 0.0;
 #pragma unroll
@@ -503,7 +667,7 @@ __global__ void __launch_bounds__(256) k_plaquette(const double* __restrict__ fu
 // each site: h links along mu, w along nu, back along mu, back along nu
 // (wilson_loop, wilsonloop.cpp:58-113)
 template <int NC>
-__global__ void __launch_bounds__(256) k_wilson_loop(const double* __restrict__ fund, int h, int w, double* partials,
+__global__ void __launch_bounds__(256) k_wilson_loop(const double2* __restrict__ fund, int h, int w, double* partials,
                                                      unsigned* ticket, double* out, Geom g) {
   int id = blockIdx.x * 256 + threadIdx.x;
   double v[1] = {0.0};
@@ -539,32 +703,6 @@ __global__ void __launch_bounds__(256) k_sumsq(const double* __restrict__ a, lon
 }
 
 // ---------------------------------------------------------------------------
-int md_init_constants(Ctx* c) {
-  int nc = c->nc, ng = nc * nc - 1;
-  std::vector<double2> h(15 * 16, make_double2(0, 0));
-  for (int a = 0; a < ng; a++) {
-    int k = 0;
-    for (int i = 0; i < nc; i++)
-      for (int j = 0; j < nc; j++) {
-        if (i > j) {
-          if (k == a) { h[a * 16 + i * nc + j].y += 1; h[a * 16 + j * nc + i].y += 1; }
-          k++;
-        } else if (i < j) {
-          if (k == a) { h[a * 16 + i * nc + j].x += 1; h[a * 16 + j * nc + i].x -= 1; }
-          k++;
-        } else if (i > 0) {
-          if (k == a) {
-            double w = sqrt(2.0 / (i * (i + 1)));
-            for (int q = 0; q < i; q++) h[a * 16 + q * nc + q].y += w;
-            h[a * 16 + i * nc + i].y -= i * w;
-          }
-          k++;
-        }
-      }
-  }
-  return upload_table(c, c->tab_itf, h.data(), h.size());
-}
-
 #define YH_NC_SWITCH(...)                                     \
   switch (c->nc) {                                            \
     case 2: { constexpr int NC_ = 2; __VA_ARGS__; } break;    \
@@ -573,13 +711,35 @@ int md_init_constants(Ctx* c) {
     default: set_error("unsupported NC"); return YH_ERR_UNSUPPORTED; \
   }
 
+template <int NC, bool TO_AOS>
+static void fund_aos_launch(Ctx* c) {
+  dim3 grid((c->g.VH + AosTile<NC>::S - 1) / AosTile<NC>::S, 2);
+  hipLaunchKernelGGL((k_fund_aos<NC, TO_AOS>), grid, dim3(256), 0, c->stream, c->fund_aos, c->fund, c->g);
+}
+
+int gauge_upload(Ctx* c, const double* host) {
+  const size_t bytes = sizeof(double) * 4 * c->g.V * 2 * c->nc * c->nc;
+  YH_HIP(hipMemcpyAsync(c->fund_aos, host, bytes, hipMemcpyHostToDevice, c->stream));
+  YH_NC_SWITCH((fund_aos_launch<NC_, false>(c)));
+  YH_HIP(hipGetLastError());
+  return YH_OK;
+}
+
+int gauge_download(Ctx* c, double* host) {
+  const size_t bytes = sizeof(double) * 4 * c->g.V * 2 * c->nc * c->nc;
+  YH_NC_SWITCH((fund_aos_launch<NC_, true>(c)));
+  YH_HIP(hipGetLastError());
+  YH_HIP(hipMemcpyAsync(host, c->fund_aos, bytes, hipMemcpyDeviceToHost, c->stream));
+  YH_HIP(hipStreamSynchronize(c->stream));
+  return YH_OK;
+}
+
 int md_gauge_force(Ctx* c, double dt, double beta) {
   int rc;
   if ((rc = force_alloc(c))) return rc;
-  double coeff = dt * beta / c->nc;
-  dim3 grid((4 * c->g.V + 127) / 128);
-  YH_NC_SWITCH(hipLaunchKernelGGL((k_gauge_force<NC_, false>), grid, dim3(128), 0, c->stream, c->fund, c->mom, coeff,
-                                  1.0, 0.0, c->g, c->tab_itf));
+  dim3 grid((c->g.VH + 63) / 64 * 8);
+  YH_NC_SWITCH(hipLaunchKernelGGL((k_wilson_force<NC_>), grid, dim3(192), 0, c->stream, c->fund, c->mom,
+                                  dt * beta / c->nc * 0.5, c->g));
   YH_HIP(hipGetLastError());
   return YH_OK;
 }
@@ -587,10 +747,9 @@ int md_gauge_force(Ctx* c, double dt, double beta) {
 int md_improved_gauge_force(Ctx* c, double dt, double beta, double c0, double c1) {
   int rc;
   if ((rc = force_alloc(c))) return rc;
-  double coeff = dt * beta / c->nc;
-  dim3 grid((4 * c->g.V + 127) / 128);
-  YH_NC_SWITCH(hipLaunchKernelGGL((k_gauge_force<NC_, true>), grid, dim3(128), 0, c->stream, c->fund, c->mom, coeff,
-                                  c0, c1, c->g, c->tab_itf));
+  dim3 grid((c->g.VH + 63) / 64 * 8);
+  YH_NC_SWITCH(hipLaunchKernelGGL((k_rect_force<NC_>), grid, dim3(64 * rect_waves(NC_)), 0, c->stream, c->fund, c->mom,
+                                  dt * beta / c->nc * 0.5, c0, c1, c->g));
   YH_HIP(hipGetLastError());
   return YH_OK;
 }
@@ -630,7 +789,7 @@ int md_apply_gauge_bcs(Ctx* c) {
       return YH_ERR_UNSUPPORTED;
     }
   }
-  dim3 grid((4 * c->g.V + 255) / 256);
+  dim3 grid((c->g.V + 255) / 256, 4);
   YH_NC_SWITCH(hipLaunchKernelGGL((k_gauge_bcs<NC_>), grid, dim3(256), 0, c->stream, c->fund, c->g, ph));
   YH_HIP(hipGetLastError());
   return YH_OK;
@@ -642,14 +801,14 @@ int md_update_links(Ctx* c, double eps) {
   // the fixed links' momenta are zeroed, so exp(0) U leaves them as they are
   // (update.cpp:231-243 zeroes them, updates, and sets the fixed links again)
   if ((rc = mom_bcs(c))) return rc;
-  dim3 grid((4 * c->g.V + 127) / 128);
+  dim3 grid((c->g.V + 127) / 128, 4);
   YH_NC_SWITCH(hipLaunchKernelGGL((k_update_links<NC_>), grid, dim3(128), 0, c->stream, c->fund, c->mom, eps, c->g));
   YH_HIP(hipGetLastError());
   return YH_OK;
 }
 
 int md_reunitarize(Ctx* c) {
-  dim3 grid((4 * c->g.V + 127) / 128);
+  dim3 grid((c->g.V + 127) / 128, 4);
   YH_NC_SWITCH(hipLaunchKernelGGL((k_reunitarize<NC_>), grid, dim3(128), 0, c->stream, c->fund, c->g));
   YH_HIP(hipGetLastError());
   return YH_OK;
@@ -726,10 +885,7 @@ int yh_get_gauge(yh_ctx* c, double* links) {
   if (!c || !links) { set_error("null argument"); return YH_ERR_ARG; }
   if (!c->gauge_set) { set_error("no gauge field"); return YH_ERR_STATE; }
   YH_HIP(hipSetDevice(c->device));
-  size_t n = (size_t)4 * c->g.V * 2 * c->nc * c->nc;
-  YH_HIP(hipMemcpyAsync(links, c->fund, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  YH_HIP(hipStreamSynchronize(c->stream));
-  return YH_OK;
+  return gauge_download(c, links);
 }
 
 int yh_represent_gauge_field(yh_ctx* c) {
