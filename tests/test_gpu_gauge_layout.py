@@ -1,11 +1,12 @@
 """The gauge kernels on lattices whose half volume is no multiple of a
 wavefront or a workgroup, against the oracle: the transposition of host links
 to component planes and back, the Wilson and improved forces, the link
-update, and the represented links and clover term built from the moved links."""
+update, the represented links and the clover term built from the moved links,
+and its inverse (log det, and the operator in every storage precision)."""
 import numpy as np
 import pytest
 
-from fields import random_gauge
+from fields import gaussian_spinor, random_gauge
 from oracle import BC_ANTIPERIODIC, BC_OPEN, Oracle
 
 pytestmark = pytest.mark.gpu
@@ -48,3 +49,14 @@ def test_ragged_lattices(model, nc, rep, dims, bc):
     assert np.abs(lat.gauge_repr().reshape(o.get_repr().shape) - o.get_repr()).max() < 1e-13
     want = o.get_clover()
     assert np.abs(lat.clover_term().reshape(want.shape) - want).max() < 1e-13 * max(1.0, np.abs(want).max())
+    mass = 0.3
+    assert abs(lat.clover_logdet(mass) - o.clover_logdet(mass)) < 1e-12 * abs(o.clover_logdet(mass))
+    src = gaussian_spinor(rng, o.V, o.dr)
+    want = np.zeros_like(src)
+    o.Hphi(mass, want, src.copy())
+    # 64-bit, 32-bit and 16-bit fixed-point storage of links, clover term and inverse
+    for prec, tol in (("f64", 1e-13), ("f32", 2e-6), ("f16", 2e-4)):
+        fs, fd = lat.field(prec).upload(src), lat.field(prec)
+        lat.Hphi(mass, fd, fs)
+        got = fd.download(yh.EVEN)[: o.VH]
+        assert np.abs(got - want[: o.VH]).max() < tol * np.abs(want).max(), prec

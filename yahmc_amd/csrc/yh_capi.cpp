@@ -429,6 +429,7 @@ int yh_destroy(yh_ctx* c) {
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   free_scratch(c);
+  c->links[PREC_F64][RECON_12] = nullptr;  // shares the 18-real planes
   for (int p = 0; p < 3; p++) {
     for (int r = 0; r < 2; r++)
       if (c->links[p][r]) (void)hipFree(c->links[p][r]);
@@ -469,7 +470,6 @@ int yh_set_gauge(yh_ctx* c, const double* links) {
   int rc;
   if ((rc = gauge_upload(c, links))) return rc;
   if ((rc = gauge_represent(c))) return rc;
-  if ((rc = gauge_derive_links(c))) return rc;
   if ((rc = clover_build(c))) return rc;
   if (c->csw != 0.0 && (rc = clover_reserve_inverse(c))) return rc;
   YH_HIP(hipStreamSynchronize(c->stream));

@@ -405,6 +405,13 @@ struct LinkStore<PREC_F16, RECON_12, D> { typedef uint2 vec; static constexpr in
 template <int D>
 struct LinkStore<PREC_F32, RECON_12H, D> { typedef uint2 vec; static constexpr int NV = 3; static constexpr int BYTES = 24; };
 
+// component planes from one direction's links to the next (FP64 12-real links
+// are the first two rows of the 18-real planes)
+template <int PREC, int RECON, int D>
+constexpr int link_planes() {
+  return PREC == PREC_F64 && RECON == RECON_12 ? D * D : LinkStore<PREC, RECON, D>::NV;
+}
+
 // third row of an SU(3) matrix from the first two: conj(r0 x r1)
 template <typename R>
 __device__ __forceinline__ Cx<R> conj_cross(Cx<R> a, Cx<R> b, Cx<R> c, Cx<R> d) {

@@ -48,7 +48,7 @@ int hop_launch(Ctx* c, const HopCall& h) {
   int lnv;
   switch (h.recon == RECON_12H ? 5 : h.prec * 2 + h.recon) {
     case 0: lvbytes = 16; lnv = c->dr * c->dr; break;
-    case 1: lvbytes = 16; lnv = 6; break;
+    case 1: lvbytes = 16; lnv = c->dr * c->dr; break;  // link_planes()
     case 2: lvbytes = 8; lnv = c->dr * c->dr; break;
     case 3: lvbytes = 16; lnv = 3; break;
     case 4: lvbytes = 4; lnv = c->dr * c->dr; break;

@@ -73,7 +73,6 @@ template <int MU, bool FWD, int D, int PREC, int RECON, typename R>
 __device__ __forceinline__ void hop_dir_src(Cx<R> (&acc)[4][D], const HopArgs& a, const void* in, const float* in_nrm,
                                             int stride, int nidx, int lidx, bool flip) {
   typedef Proj<MU, FWD> P;
-  constexpr int LNV = LinkStore<PREC, RECON, D>::NV;
   typedef typename LinkStore<PREC, RECON, D>::vec LV;
   Cx<R> s[4][D];
   R sc = (R)1;
@@ -85,7 +84,7 @@ __device__ __forceinline__ void hop_dir_src(Cx<R> (&acc)[4][D], const HopArgs& a
     h[0][i] = s[2][i] + unit_mul<P::PC0>(s[P::PI0][i]);
     h[1][i] = s[3][i] + unit_mul<P::PC1>(s[P::PI1][i]);
   }
-  const LV* lbase = (const LV*)(FWD ? a.lf : a.lb) + (size_t)MU * LNV * a.g.VHpad;
+  const LV* lbase = (const LV*)(FWD ? a.lf : a.lb) + (size_t)MU * link_planes<PREC, RECON, D>() * a.g.VHpad;
   Cx<R> r[2][D];
   if constexpr (PREC == PREC_F64 && RECON == RECON_18 && D >= 6) {
     // a D_R x D_R FP64 link is 2 D_R^2 doubles (144 registers at D_R = 6,

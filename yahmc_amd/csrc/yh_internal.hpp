@@ -139,9 +139,8 @@ int field_convert(Ctx* c, Field* dst, int dpar, const Field* src, int spar);
 int gauge_init_basis(Ctx* c);
 int gauge_upload(Ctx* c, const double* host);    // host links (4V suNg) -> fund
 int gauge_download(Ctx* c, double* host);        // fund -> host links
-int gauge_represent(Ctx* c);                 // fund -> F64 R18 links
-int gauge_derive_links(Ctx* c);              // F64 R18 -> other precisions
-int clover_build(Ctx* c);                    // packed FP64 clover
+int gauge_represent(Ctx* c);                 // fund -> represented links, every precision
+int clover_build(Ctx* c);                    // packed clover term, every precision
 int clover_invert(Ctx* c, double sigma);     // odd-site inverses (+ logdet)
 int clover_reserve_inverse(Ctx* c);          // allocate the inverse buffers once
 int clover_logdet_sum(Ctx* c, double* out);

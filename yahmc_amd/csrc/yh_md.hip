@@ -894,7 +894,6 @@ int yh_represent_gauge_field(yh_ctx* c) {
   YH_HIP(hipSetDevice(c->device));
   int rc;
   if ((rc = gauge_represent(c))) return rc;
-  if ((rc = gauge_derive_links(c))) return rc;
   if ((rc = clover_build(c))) return rc;
   return md_sync(c, YH_OK);
 }
