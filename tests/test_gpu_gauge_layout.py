@@ -60,3 +60,38 @@ def test_ragged_lattices(model, nc, rep, dims, bc):
         lat.Hphi(mass, fd, fs)
         got = fd.download(yh.EVEN)[: o.VH]
         assert np.abs(got - want[: o.VH]).max() < tol * np.abs(want).max(), prec
+
+
+FORCE_MODELS = [("su2_fund", 2, "fundamental"), ("su3_fund", 3, "fundamental"), ("su4_asym", 4, "antisymmetric"),
+                ("su3_sym", 3, "symmetric")]
+
+
+@pytest.mark.parametrize("model,nc,rep", FORCE_MODELS)
+@pytest.mark.parametrize("dims,bc", [((4, 2, 6, 6), "antiperiodic"), ((6, 4, 6, 10), "open")])
+def test_ragged_fermion_forces(model, nc, rep, dims, bc):
+    """The force sequence of a two-flavour monomial (packed clover-force
+    matrices up to D_R = 4, full ones at 6), and the matrices themselves."""
+    print(f"\n[case] fermion forces {model} {dims} {bc}", flush=True)
+    o = Oracle(model).init(dims, bc=BC_OPEN if bc == "open" else BC_ANTIPERIODIC, csw=1.0)
+    rng = np.random.default_rng(72)
+    links = random_gauge(rng, o.V, nc)
+    P = rng.normal(size=(4 * o.V, nc * nc - 1))
+    o.set_gauge(links)
+    o.apply_bcs_on_gauge()
+    o.represent()
+    lat = yh.Lattice(dims, nc=nc, repr=rep, bc=bc, csw=1.0)
+    lat.set_gauge(o.get_gauge())
+    src = gaussian_spinor(rng, o.V, o.dr)
+    field = lat.field("f64").upload(src)
+    for x, y in ((o, src.copy()), (lat, field)):
+        x.set_momenta(P)
+        x.begin_fermion_force()
+        x.wilson_fermion_force_q(0.3, 0.2, 1.0, y)
+        x.clover_logdet_force(0.2, 2.0)
+    want = o.get_clover_force()
+    got = lat.get_clover_force().reshape(want.shape)
+    assert np.abs(got - want).max() < 1e-12 * np.abs(want).max()
+    for x in (o, lat):
+        x.end_fermion_force(0.3)
+    got, want = lat.get_momenta(), o.get_momenta()
+    assert np.abs(got - want).max() < 1e-12 * np.abs(want).max()

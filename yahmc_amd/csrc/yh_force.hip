@@ -9,10 +9,13 @@
 // algebra_project      : library/suNa.cpp:102-111 (TF = 2)
 //
 // Device layouts: momenta mom[(mu * NG + a) * V + id] (FP64, id = full EO
-// index), clover force matrices clf[(plane * D * D + e) * V + id] (double2),
-// planes in the reference order 01, 02, 12, 03, 13, 23.
+// index).  The clover force matrices are anti-Hermitian; planes in the
+// reference order 01, 02, 12, 03, 13, 23.  D_R <= 4 keeps their D^2 reals,
+// clf[(plane * D * D + e) * V + id] (double): Im of the diagonal, then re, im
+// of the lower triangle row by row, half the bytes of every pass over them;
+// D_R >= 6 keeps full matrices (double2), whose rows k_force_clover_x reads.
 #include <vector>
-#include <mutex>
+#include <type_traits>
 #include <utility>
 #include "yh_internal.hpp"
 
@@ -20,8 +23,7 @@ namespace yh {
 
 // represented generators iT^R_a, a < NG, D x D row-major: the context's
 // table tab_itr[(a * D + i) * D + k], passed to the kernels
-__constant__ double2 c_g5omg[4 * 16];    // gamma5 (1 - gamma_mu)
-__constant__ double2 c_g5sig[6 * 16];    // gamma5 (1/2)[gamma_mu, gamma_nu], reference plane order
+constexpr int kClfPacked = 4;            // D_R up to which the clover force matrices are packed
 
 typedef Cx<double> cd;
 
@@ -110,57 +112,13 @@ static void rep_generators(int nc, int repr, int dr, std::vector<cd>& out) {
   }
 }
 
-// chiral gamma basis as applied by library/spinor.cpp:191-264
-static void gamma_mats(cd g[4][4][4]) {
-  for (int m = 0; m < 4; m++)
-    for (int a = 0; a < 4; a++)
-      for (int b = 0; b < 4; b++) g[m][a][b] = cd(0, 0);
-  g[0][0][2] = g[0][1][3] = g[0][2][0] = g[0][3][1] = cd(-1, 0);
-  g[1][0][3] = g[1][1][2] = cd(0, -1);
-  g[1][2][1] = g[1][3][0] = cd(0, 1);
-  g[2][0][3] = cd(-1, 0); g[2][1][2] = cd(1, 0); g[2][2][1] = cd(1, 0); g[2][3][0] = cd(-1, 0);
-  g[3][0][2] = cd(0, -1); g[3][1][3] = cd(0, 1); g[3][2][0] = cd(0, 1); g[3][3][1] = cd(0, -1);
-}
-
 int force_init_constants(Ctx* c) {
   std::vector<cd> itr;
   rep_generators(c->nc, c->repr, c->dr, itr);
   std::vector<double2> h(TAB_ITR, make_double2(0, 0));
   if (itr.size() > h.size()) { set_error("generator table too small"); return YH_ERR_UNSUPPORTED; }
   for (size_t i = 0; i < itr.size(); i++) h[i] = make_double2(itr[i].re, itr[i].im);
-  int rc = upload_table(c, c->tab_itr, h.data(), h.size());
-  if (rc) return rc;
-  // gamma5 (1 - gamma_mu) and gamma5 sigma_mu_nu do not depend on the model:
-  // uploaded once per device
-  static std::mutex mtx;
-  static unsigned done_mask = 0;
-  std::lock_guard<std::mutex> lk(mtx);
-  if (c->device < 32 && (done_mask >> c->device) & 1u) return YH_OK;
-  cd g[4][4][4];
-  gamma_mats(g);
-  const double g5[4] = {1, 1, -1, -1};
-  std::vector<double2> om(4 * 16), sg(6 * 16);
-  for (int m = 0; m < 4; m++)
-    for (int a = 0; a < 4; a++)
-      for (int b = 0; b < 4; b++) {
-        cd v = cd(a == b ? 1.0 : 0.0, 0) - g[m][a][b];
-        om[m * 16 + a * 4 + b] = make_double2(g5[a] * v.re, g5[a] * v.im);
-      }
-  const int planes[6][2] = {{0, 1}, {0, 2}, {1, 2}, {0, 3}, {1, 3}, {2, 3}};
-  for (int k = 0; k < 6; k++) {
-    int mu = planes[k][0], nu = planes[k][1];
-    for (int a = 0; a < 4; a++)
-      for (int b = 0; b < 4; b++) {
-        cd s(0, 0);
-        for (int q = 0; q < 4; q++) s = s + g[mu][a][q] * g[nu][q][b] - g[nu][a][q] * g[mu][q][b];
-        sg[k * 16 + a * 4 + b] = make_double2(g5[a] * 0.5 * s.re, g5[a] * 0.5 * s.im);
-      }
-  }
-  YH_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_g5omg), om.data(), sizeof(double2) * om.size()));
-  YH_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_g5sig), sg.data(), sizeof(double2) * sg.size()));
-  YH_HIP(hipDeviceSynchronize());
-  if (c->device < 32) done_mask |= 1u << c->device;
-  return YH_OK;
+  return upload_table(c, c->tab_itr, h.data(), h.size());
 }
 
 // ---------------------------------------------------------------------------
@@ -171,19 +129,9 @@ struct FF {
   const void* y[2];   // rhs halves (FP64)
 };
 
-__device__ __forceinline__ int fidx(int t, int x, int y, int z, const Geom& g) {
-  return ((t + x + y + z) & 1) * g.VH + half_index(t, x, y, z, g);
-}
-
 __device__ __forceinline__ void fcoords(int id, const Geom& g, int c[4]) {
   int p = id >= g.VH;
   site_coords(id - p * g.VH, p, g, c);
-}
-
-__device__ __forceinline__ int fshift(const int c[4], int mu, int d, const Geom& g) {
-  int n[4] = {c[0], c[1], c[2], c[3]};
-  n[mu] = (n[mu] + d + g.L[mu]) % g.L[mu];
-  return fidx(n[0], n[1], n[2], n[3], g);
 }
 
 // spinor of site id; zero on the time slices the open and SF boundaries
@@ -203,72 +151,6 @@ __device__ __forceinline__ void load_full_spinor(cd (&s)[4][D], const void* cons
         for (int i = 0; i < D; i++) s[a][i] = cd(0, 0);
     }
   }
-}
-
-// represented link U_R(id, mu) with the antiperiodic sign of the reference's
-// gfield_repr (library/bcs.cpp:264-272)
-template <int D>
-__device__ __forceinline__ void load_link_bc(cd (&u)[D][D], const double2* links, int id, int mu, const Geom& g) {
-  int p = id >= g.VH, k = id - p * g.VH;
-  const double2* base = links + (size_t)(p * 4 + mu) * D * D * g.VHpad;
-#pragma unroll
-  for (int e = 0; e < D * D; e++) {
-    double2 v = base[(size_t)e * g.VHpad + k];
-    u[e / D][e % D] = cd(v.x, v.y);
-  }
-  if (g.bc == BC_ANTIPERIODIC && mu == 0) {
-    int c[4];
-    site_coords(k, p, g, c);
-    if (c[0] == 0) {
-#pragma unroll
-      for (int i = 0; i < D; i++)
-#pragma unroll
-        for (int j = 0; j < D; j++) u[i][j] = cd(-u[i][j].re, -u[i][j].im);
-    }
-  }
-}
-
-template <int D>
-__device__ __forceinline__ void spin_mat(cd (&o)[4][D], const double2* M, const cd (&s)[4][D]) {
-#pragma unroll
-  for (int a = 0; a < 4; a++)
-#pragma unroll
-    for (int c = 0; c < D; c++) {
-      cd v(0, 0);
-#pragma unroll
-      for (int b = 0; b < 4; b++) {
-        double2 m = M[a * 4 + b];
-        if (m.x != 0.0 || m.y != 0.0) cmac(v, cd(m.x, m.y), s[b][c]);
-      }
-      o[a][c] = v;
-    }
-}
-
-// F_ij += sum_spin a_i conj(b_j)
-template <int D>
-__device__ __forceinline__ void outer_acc(cd (&F)[D][D], const cd (&a)[4][D], const cd (&b)[4][D]) {
-#pragma unroll
-  for (int i = 0; i < D; i++)
-#pragma unroll
-    for (int j = 0; j < D; j++)
-#pragma unroll
-      for (int s = 0; s < 4; s++) {
-        F[i][j].re += a[s][i].re * b[s][j].re + a[s][i].im * b[s][j].im;
-        F[i][j].im += a[s][i].im * b[s][j].re - a[s][i].re * b[s][j].im;
-      }
-}
-
-template <int D>
-__device__ __forceinline__ void mmul(cd (&R)[D][D], const cd (&A)[D][D], const cd (&B)[D][D]) {
-#pragma unroll
-  for (int i = 0; i < D; i++)
-#pragma unroll
-    for (int j = 0; j < D; j++) {
-      cd s(0, 0);
-#pragma unroll
-      for (int k = 0; k < D; k++) cmac(s, A[i][k], B[k][j]);
-      R[i][j] = s;
-    }
 }
 
 // mom_a += -(coeff / TF) Re Tr(iT^R_a F)
@@ -319,12 +201,6 @@ __device__ __forceinline__ MSrc link_src(const double2* links, int id, int mu, b
   return MSrc{links + (size_t)(p * 4 + mu) * D * D * g.VHpad + k, (size_t)g.VHpad, sgn, dag};
 }
 
-// clover-force matrix of plane `num` at site id
-template <int D>
-__device__ __forceinline__ MSrc clf_src(const double2* clf, int num, int id, int V) {
-  return MSrc{clf + (size_t)num * D * D * V + id, (size_t)V, 1.0, false};
-}
-
 // the same source, but readable only after `dep` is final: every element of
 // dep passes through an empty volatile asm and the pointer through one more,
 // so the compiler can neither hoist the reads above the computation of dep
@@ -341,14 +217,6 @@ __device__ __forceinline__ MSrc after(MSrc m, cd (&dep)[D][D]) {
     }
   __asm__ volatile("" : "+v"(m.p));
   return m;
-}
-
-template <int D>
-__device__ __forceinline__ void mload(cd (&A)[D][D], const MSrc& m) {
-#pragma unroll
-  for (int i = 0; i < D; i++)
-#pragma unroll
-    for (int j = 0; j < D; j++) A[i][j] = mget<D>(m, i, j);
 }
 
 // C (+)= s * M B, M in memory
@@ -370,93 +238,192 @@ __device__ __forceinline__ void mul_mb(cd (&C)[D][D], const MSrc& M, const cd (&
   }
 }
 
-// C (+)= s * A M, M in memory
-template <int D, bool ACC>
-__device__ __forceinline__ void mul_am(cd (&C)[D][D], const cd (&A)[D][D], const MSrc& M, double s) {
-#pragma unroll
-  for (int j = 0; j < D; j++) {
-    cd col[D];
-#pragma unroll
-    for (int i = 0; i < D; i++) col[i] = cd(0, 0);
-#pragma unroll
-    for (int k = 0; k < D; k++) {
-      const cd m = mget<D>(M, k, j);
-#pragma unroll
-      for (int i = 0; i < D; i++) cmac(col[i], A[i][k], m);
-    }
-#pragma unroll
-    for (int i = 0; i < D; i++) C[i][j] = ACC ? C[i][j] + s * col[i] : s * col[i];
-  }
-}
-
 // ---------------------------------------------------------------------------
 // kernels
 // ---------------------------------------------------------------------------
-// hopping force, one thread per (site, mu)  (forces.cpp:204-223)
+// a product of chiral-basis gammas (library/spinor.cpp:191-264) as one entry
+// per row: (g psi)_a = i^pow[a] psi_{col[a]}
+struct SpinPerm {
+  int col[4], pow[4];
+};
+constexpr SpinPerm gamma_perm(int mu) {
+  return mu == 0   ? SpinPerm{{2, 3, 0, 1}, {2, 2, 2, 2}}
+         : mu == 1 ? SpinPerm{{3, 2, 1, 0}, {3, 3, 1, 1}}
+         : mu == 2 ? SpinPerm{{3, 2, 1, 0}, {2, 0, 0, 2}}
+                   : SpinPerm{{2, 3, 0, 1}, {3, 1, 1, 3}};
+}
+// gamma5 sigma_{mu nu} = gamma5 gamma_mu gamma_nu of plane k (mu < nu)
+constexpr SpinPerm g5sigma_perm(int k) {
+  const int mu = k == 0 || k == 1 || k == 3 ? 0 : k == 5 ? 2 : 1, nu = k == 0 ? 1 : k < 3 ? 2 : 3;
+  const SpinPerm m = gamma_perm(mu), n = gamma_perm(nu);
+  SpinPerm r{};
+  for (int a = 0; a < 4; a++) {
+    r.col[a] = n.col[m.col[a]];
+    r.pow[a] = (m.pow[a] + n.pow[m.col[a]] + (a >= 2 ? 2 : 0)) % 4;
+  }
+  return r;
+}
+// multiplication by i^P
+template <int P>
+__device__ __forceinline__ cd ipow(cd z) {
+  return unit_mul<P == 0 ? 0 : P == 1 ? 2 : P == 2 ? 1 : 3>(z);
+}
+
+// F += sum_spin [g5 (1 - g_mu) n] o^+ for a neighbour's spinor n and the own
+// spinor o.  1 - g_mu has rank two: its lower rows are
+// h_k = n_{2+k} - i^pow n_col and its upper rows multiples of them, so the
+// sum is h_k times (a combination of o_{2+k} and the upper row's o)^+, k = 0, 1.
+template <int MU, int D, typename Load>
+__device__ __forceinline__ void hop_outer(cd (&F)[D][D], Load&& neigh, Load&& own) {
+  constexpr SpinPerm G = gamma_perm(MU);
+  auto spin = [&](auto kc) {
+    constexpr int k = kc(), j = G.col[2 + k];  // the upper row that is a multiple of h_k
+    cd h[D], o[D];
+#pragma unroll
+    for (int i = 0; i < D; i++) {
+      const cd a = ipow<(G.pow[2 + k] + 2) % 4>(neigh(j, i)), b = ipow<(6 - G.pow[j]) % 4>(own(j, i));
+      h[i] = neigh(2 + k, i) + a;
+      o[i] = b - own(2 + k, i);
+    }
+#pragma unroll
+    for (int i = 0; i < D; i++)
+#pragma unroll
+      for (int m = 0; m < D; m++) {
+        F[i][m].re = fma(h[i].re, o[m].re, fma(h[i].im, o[m].im, F[i][m].re));
+        F[i][m].im = fma(h[i].im, o[m].re, fma(-h[i].re, o[m].im, F[i][m].im));
+      }
+  };
+  spin(std::integral_constant<int, 0>());
+  spin(std::integral_constant<int, 1>());
+}
+
+// hopping force (forces.cpp:204-223), one thread per (site, mu): a workgroup
+// takes 64 consecutive sites of one parity, one wave per mu, so that each
+// load is a whole segment of a component plane and the four mu share the
+// site's own spinors
 template <int NG, int D>
 __global__ void __launch_bounds__(256) k_force_hop(FF f, const double2* __restrict__ links, double* __restrict__ mom,
                                                    double coeff, Geom g, const double2* __restrict__ itr) {
-  int t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= 4 * g.V) return;
-  int id = t >> 2, mu = t & 3;
-  int c[4];
-  fcoords(id, g, c);
-  int fw = fshift(c, mu, 1, g);
+  const int bl = xcd_block(gridDim.x, 64);
+  const int p = bl & 1, k = (bl >> 1) * 64 + (threadIdx.x & 63);
+  const int mu = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (k >= g.VH) return;
+  const int id = p * g.VH + k;
+  int c[4], cf[4];
+  site_coords(k, p, g, c);
+  const int kf = neighbour(c, mu, 1, g, cf) - (1 - p) * g.VH;  // half index of x + mu
+  // the slices that the open and SF boundaries clear (load_full_spinor)
+  const bool zx = bc_zero_slice(c[0], g), zf = bc_zero_slice(cf[0], g);
+  struct Get {
+    const double2* p;
+    size_t s;
+    bool zero;
+    __device__ __forceinline__ cd operator()(int spin, int i) const {
+      const double2 v = p[(size_t)(spin * D + i) * s];
+      return zero ? cd(0, 0) : cd(v.x, v.y);
+    }
+  };
   cd F[D][D];
 #pragma unroll
   for (int i = 0; i < D; i++)
 #pragma unroll
     for (int j = 0; j < D; j++) F[i][j] = cd(0, 0);
-  {
-    cd s[4][D], ps[4][D], o[4][D];
-    load_full_spinor<D>(s, f.x, fw, g);          // lhs(x + mu)
-    spin_mat<D>(ps, c_g5omg + mu * 16, s);
-    load_full_spinor<D>(o, f.y, id, g);          // rhs(x)
-    outer_acc<D>(F, ps, o);
-    // the second pair of spinors is read after F is updated (fewer live registers)
-    const MSrc nf = after<D>(MSrc{nullptr, 0, 1.0, false}, F);
-    const int z = (int)(size_t)nf.p;
-    load_full_spinor<D>(s, f.y, fw + z, g);      // rhs(x + mu)
-    spin_mat<D>(ps, c_g5omg + mu * 16, s);
-    load_full_spinor<D>(o, f.x, id, g);          // lhs(x)
-    outer_acc<D>(F, ps, o);
+  const size_t S = g.VHpad;
+  const void* const(&x)[2] = f.x;
+  const void* const(&y)[2] = f.y;
+#pragma unroll
+  for (int half = 0; half < 2; half++) {
+    // lhs(x + mu) with rhs(x), then rhs(x + mu) with lhs(x); the second pair
+    // is read after F is updated (fewer live registers)
+    const int z = half ? (int)(size_t)after<D>(MSrc{nullptr, 0, 1.0, false}, F).p : 0;
+    const Get n{(const double2*)(half ? y : x)[1 - p] + kf + z, S, zf};
+    const Get o{(const double2*)(half ? x : y)[p] + k + z, S, zx};
+    switch (mu) {
+      case 0: hop_outer<0, D>(F, n, o); break;
+      case 1: hop_outer<1, D>(F, n, o); break;
+      case 2: hop_outer<2, D>(F, n, o); break;
+      default: hop_outer<3, D>(F, n, o); break;
+    }
   }
   cd R[D][D];
   mul_mb<D, false>(R, after<D>(link_src<D>(links, id, mu, false, g), F), F, 1.0);
   project_add<NG, D>(mom, mu, id, g.V, R, coeff, itr);
 }
 
-// clover force matrices, one thread per site  (forces.cpp:130-168)
-template <int D>
-__global__ void __launch_bounds__(256) k_force_clover_site(FF f, double2* __restrict__ clf, double residue, Geom g) {
+// clover force matrices, one thread per site  (forces.cpp:130-168):
+// F = sum_spin (S X) Y^+ + (S Y) X^+ with S = gamma5 sigma anti-Hermitian, so
+// F = M - M^+ with M = sum_spin (S X) Y^+.  Packed matrices (PACK): M once
+// and D^2 reals read and written, 741 -> 240 us at 32^4 for SU(3).
+template <int D, bool PACK>
+__global__ void __launch_bounds__(256) k_force_clover_site(FF f, double* __restrict__ clf, double residue, Geom g) {
   int id = blockIdx.x * 256 + threadIdx.x;
   if (id >= g.V) return;
   cd X[4][D], Y[4][D];
   load_full_spinor<D>(X, f.x, id, g);
   load_full_spinor<D>(Y, f.y, id, g);
-  for (int k = 0; k < 6; k++) {
-    cd sx[4][D], sy[4][D], F[D][D];
+  auto plane = [&](auto kc) {
+    constexpr int k = kc();
+    constexpr SpinPerm S = g5sigma_perm(k);
+    // entry (i, j) of M
+    auto m = [&](int i, int j) -> cd {
+      cd v(0, 0);
+      auto spin = [&](auto ac) {
+        constexpr int a = ac();
+        const cd x = ipow<S.pow[a]>(X[S.col[a]][i]);
+        const cd y = Y[a][j];
+        v.re = fma(x.re, y.re, fma(x.im, y.im, v.re));
+        v.im = fma(x.im, y.re, fma(-x.re, y.im, v.im));
+      };
+      spin(std::integral_constant<int, 0>());
+      spin(std::integral_constant<int, 1>());
+      spin(std::integral_constant<int, 2>());
+      spin(std::integral_constant<int, 3>());
+      return v;
+    };
+    if constexpr (PACK) {
+      double* q = clf + (size_t)k * D * D * g.V + id;
+      int e = D;
 #pragma unroll
-    for (int i = 0; i < D; i++)
+      for (int i = 0; i < D; i++) {
+        const cd v = m(i, i);
+        q[(size_t)i * g.V] = fma(2.0 * residue, v.im, q[(size_t)i * g.V]);
 #pragma unroll
-      for (int j = 0; j < D; j++) F[i][j] = cd(0, 0);
-    spin_mat<D>(sx, c_g5sig + k * 16, X);
-    spin_mat<D>(sy, c_g5sig + k * 16, Y);
-    outer_acc<D>(F, sx, Y);  // (g5 sigma lhs) # rhs
-    outer_acc<D>(F, sy, X);  // (g5 sigma rhs) # lhs
+        for (int j = 0; j < i; j++) {
+          const cd u = m(i, j), w = m(j, i);
+          q[(size_t)e * g.V] = fma(residue, u.re - w.re, q[(size_t)e * g.V]);
+          q[(size_t)(e + 1) * g.V] = fma(residue, u.im + w.im, q[(size_t)(e + 1) * g.V]);
+          e += 2;
+        }
+      }
+    } else {
+      double2* q = (double2*)clf + (size_t)k * D * D * g.V + id;
 #pragma unroll
-    for (int e = 0; e < D * D; e++) {
-      double2* p = clf + (size_t)(k * D * D + e) * g.V + id;
-      double2 v = *p;
-      *p = make_double2(v.x + residue * F[e / D][e % D].re, v.y + residue * F[e / D][e % D].im);
+      for (int i = 0; i < D; i++)
+#pragma unroll
+        for (int j = 0; j <= i; j++) {
+          const cd u = m(i, j), w = i == j ? u : m(j, i);
+          const cd v(residue * (u.re - w.re), residue * (u.im + w.im));
+          double2 z = q[(size_t)(i * D + j) * g.V];
+          q[(size_t)(i * D + j) * g.V] = make_double2(z.x + v.re, z.y + v.im);
+          if (i != j) {
+            z = q[(size_t)(j * D + i) * g.V];
+            q[(size_t)(j * D + i) * g.V] = make_double2(z.x - v.re, z.y + v.im);
+          }
+        }
     }
-  }
+  };
+  plane(std::integral_constant<int, 0>());
+  plane(std::integral_constant<int, 1>());
+  plane(std::integral_constant<int, 2>());
+  plane(std::integral_constant<int, 3>());
+  plane(std::integral_constant<int, 4>());
+  plane(std::integral_constant<int, 5>());
 }
 
 // log-det force: coeff * (sigma + clover)^-1 per odd site -> six plane
 // combinations (clover.cpp:184-262); the inverse is the stored explicit one
 template <int D>
-__global__ void __launch_bounds__(128) k_force_logdet(const double2* __restrict__ inv, double2* __restrict__ clf,
+__global__ void __launch_bounds__(128) k_force_logdet(const double2* __restrict__ inv, double* __restrict__ clf,
                                                       double coeff, Geom g) {
   int k = blockIdx.x * 128 + threadIdx.x;
   if (k >= g.VH) return;
@@ -479,8 +446,9 @@ __global__ void __launch_bounds__(128) k_force_logdet(const double2* __restrict_
     im = ((o + 1) & 1) ? w1.y : w1.x;
     return lower ? cd(coeff * re, coeff * im) : cd(coeff * re, -coeff * im);
   };
+  constexpr bool PACK = D <= kClfPacked;
   for (int i = 0; i < D; i++)
-    for (int j = 0; j < D; j++) {
+    for (int j = 0; j < (PACK ? i + 1 : D); j++) {
       cd a21 = get(0, i + D, j), a12 = conj(get(0, j + D, i));
       cd a43 = get(1, i + D, j), a34 = conj(get(1, j + D, i));
       cd a11, a22, a33, a44;
@@ -499,41 +467,22 @@ __global__ void __launch_bounds__(128) k_force_logdet(const double2* __restrict_
       xs[4] = cd(a12.re - a21.re + a34.re - a43.re, a12.im - a21.im + a34.im - a43.im);   // X_13
       xs[5] = cd(-a12.im - a21.im - a34.im - a43.im, a12.re + a21.re + a34.re + a43.re);  // X_23
       for (int q = 0; q < 6; q++) {
-        double2* p = clf + (size_t)(q * D * D + i * D + j) * g.V + id;
-        double2 v = *p;
-        *p = make_double2(v.x + xs[q].re, v.y + xs[q].im);
+        if constexpr (PACK) {
+          const int e = i == j ? i : D + i * (i - 1) + 2 * j;
+          double* p = clf + (size_t)(q * D * D + e) * g.V + id;
+          if (i == j) {
+            p[0] += xs[q].im;
+          } else {
+            p[0] += xs[q].re;
+            p[g.V] += xs[q].im;
+          }
+        } else {
+          double2* p = (double2*)clf + (size_t)(q * D * D + i * D + j) * g.V + id;
+          double2 v = *p;
+          *p = make_double2(v.x + xs[q].re, v.y + xs[q].im);
+        }
       }
     }
-}
-
-template <int D>
-__device__ __forceinline__ void load_clf(cd (&Z)[D][D], const double2* clf, int num, int id, int V) {
-#pragma unroll
-  for (int e = 0; e < D * D; e++) {
-    double2 v = clf[(size_t)(num * D * D + e) * V + id];
-    Z[e / D][e % D] = cd(v.x, v.y);
-  }
-}
-
-template <int D>
-__device__ __forceinline__ void dag(cd (&A)[D][D]) {
-  cd T[D][D];
-#pragma unroll
-  for (int i = 0; i < D; i++)
-#pragma unroll
-    for (int j = 0; j < D; j++) T[i][j] = conj(A[j][i]);
-#pragma unroll
-  for (int i = 0; i < D; i++)
-#pragma unroll
-    for (int j = 0; j < D; j++) A[i][j] = T[i][j];
-}
-
-template <int D>
-__device__ __forceinline__ void madd(cd (&A)[D][D], const cd (&B)[D][D], double s) {
-#pragma unroll
-  for (int i = 0; i < D; i++)
-#pragma unroll
-    for (int j = 0; j < D; j++) A[i][j] = A[i][j] + s * B[i][j];
 }
 
 // clover-leaf derivative (forces.cpp:33-106).  With the links
@@ -543,6 +492,16 @@ __device__ __forceinline__ void madd(cd (&A)[D][D], const cd (&B)[D][D], double 
 // x, x+mu, x-nu, x+mu-nu, x+mu+nu, x+nu:
 //   F = U(x, mu) [W8 Z0 + Z1 W8 - W5 (W0 Z2 W1 + Z3 W6) + (W2 Z4 W3 + W7 Z5) W4]
 // and P(x, mu) += proj(F, sign c_sw dt / 8).
+//
+// k_force_clover_nu (D_R <= 4): a workgroup takes 64 consecutive sites of one
+// parity and one mu, one wave per nu, as the gauge force does; a lane holds
+// whole matrices.  With A = W2, B = W3, C = W4 (above) and A = W5, B = W0,
+// C = W1 (below) both sides are the path A B C with a Z at each corner:
+//   F = W8 Z0 + Z1 W8 + [A (B Z5 C + Z4 B C)]_up - [A (B Z2 C + Z3 B C)]_down,
+//   W8 = (A B C)_up - (A B C)_down
+// (14 products); the three nu add in LDS and wave 0 projects U F.  The
+// antiperiodic signs drop out: U(x, mu) and the links of each path close a
+// plaquette, whose two time links carry the same sign.
 //
 // k_force_clover_x: the three nu of one (x, mu) in one pass (the sign folded
 // into F, one projection per (x, mu)), with the reference's association of
@@ -572,6 +531,133 @@ __device__ __forceinline__ void madd(cd (&A)[D][D], const cd (&B)[D][D], double 
 // no barrier, only the waits and compiler fences.  Work items run mu
 // fastest, each XCD taking a contiguous slab of the lattice (xcd_block), so
 // the four mu of a site share its links and clover-force matrices in L2.
+
+// M = s * (anti-Hermitian packed matrix in memory)
+template <int D>
+__device__ __forceinline__ void load_clf(cd (&Z)[D][D], const double* clf, int num, int id, int V) {
+  const double* q = clf + (size_t)num * D * D * V + id;
+  int e = D;
+#pragma unroll
+  for (int i = 0; i < D; i++) {
+    Z[i][i] = cd(0.0, q[(size_t)i * V]);
+#pragma unroll
+    for (int j = 0; j < i; j++) {
+      const double re = q[(size_t)e * V], im = q[(size_t)(e + 1) * V];
+      e += 2;
+      Z[i][j] = cd(re, im);
+      Z[j][i] = cd(-re, im);
+    }
+  }
+}
+
+// R (+)= A B
+template <int D, bool ACC>
+__device__ __forceinline__ void mmac(cd (&R)[D][D], const cd (&A)[D][D], const cd (&B)[D][D], double s = 1.0) {
+#pragma unroll
+  for (int i = 0; i < D; i++)
+#pragma unroll
+    for (int j = 0; j < D; j++) {
+      cd v(0, 0);
+#pragma unroll
+      for (int k = 0; k < D; k++) cmac(v, A[i][k], B[k][j]);
+      R[i][j] = ACC ? cd(fma(s, v.re, R[i][j].re), fma(s, v.im, R[i][j].im)) : cd(s * v.re, s * v.im);
+    }
+}
+
+// an opaque zero once every element of m is final: indices it is added to are
+// loaded after m
+template <int D>
+__device__ __forceinline__ int settled(cd (&m)[D][D]) {
+#pragma unroll
+  for (int i = 0; i < D; i++)
+#pragma unroll
+    for (int j = 0; j < D; j++) __asm__ volatile("" : "+v"(m[i][j].re), "+v"(m[i][j].im));
+  int z;
+  __asm__ volatile("v_mov_b32 %0, 0" : "=v"(z));
+  return z;
+}
+
+template <int NG, int D>
+__global__ void __launch_bounds__(192) k_force_clover_nu(const double* __restrict__ clf,
+                                                         const double2* __restrict__ links, double* __restrict__ mom,
+                                                         double coeff, Geom g, const double2* __restrict__ itr) {
+  __shared__ double2 ex[2][D * D][64];
+  // mu fastest, then parity, then site blocks; 64 workgroups per XCD in turn
+  const int b = xcd_block(gridDim.x, 64);
+  const int mu = b & 3, p = (b >> 2) & 1;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int k = (b >> 3) * 64 + lane;
+  const int kk = min(k, g.VH - 1);  // lanes past the end compute on the last site and write nothing
+  const int id = p * g.VH + kk, nu = w + (w >= mu);
+  const int hi = max(mu, nu), lo = min(mu, nu), num = hi * (hi - 1) / 2 + lo;
+  const double sign = mu < nu ? 1.0 : -1.0;
+  int c[4], cn[4], cb[4], q[4];
+  site_coords(kk, p, g, c);
+  const int om = neighbour(c, mu, 1, g, q);
+  const int on = neighbour(c, nu, 1, g, cn), omn = neighbour(cn, mu, 1, g, q);
+  const int bn = neighbour(c, nu, -1, g, cb), bmn = neighbour(cb, mu, 1, g, q);
+  auto L = [&](cd (&u)[D][D], int i, int d, bool dg) {
+    const int pp = i >= g.VH;
+    const double2* s = links + (size_t)(pp * 4 + d) * D * D * g.VHpad + (i - pp * g.VH);
+#pragma unroll
+    for (int e = 0; e < D * D; e++) {
+      const double2 v = s[(size_t)e * g.VHpad];
+      if (dg) u[e % D][e / D] = cd(v.x, -v.y);
+      else u[e / D][e % D] = cd(v.x, v.y);
+    }
+  };
+  cd F[D][D], W8[D][D];
+  // one side: F (+)= s A (B Zc C + Zb B C), W8 (+)= s A B C
+  auto side = [&](auto up, int z) {
+    constexpr bool UP = up();
+    const double s = UP ? 1.0 : -1.0;
+    cd B[D][D], C[D][D], Z[D][D], T[D][D], BC[D][D];
+    L(C, (UP ? id : bn) + z, nu, UP);
+    load_clf<D>(Z, clf, num, (UP ? on : bn) + z, g.V);  // Z5 / Z2
+    mmac<D, false>(T, Z, C);
+    L(B, (UP ? on : bn) + z, mu, true);
+    mmac<D, false>(BC, B, C);
+    mmac<D, false>(C, B, T);
+    z += settled<D>(C);
+    load_clf<D>(Z, clf, num, (UP ? omn : bmn) + z, g.V);  // Z4 / Z3
+    mmac<D, true>(C, Z, BC);
+    L(B, (UP ? om : bmn) + z, nu, !UP);
+    mmac<D, !UP>(F, B, C, s);
+    mmac<D, !UP>(W8, B, BC, s);
+  };
+  side(std::integral_constant<bool, true>(), 0);
+  side(std::integral_constant<bool, false>(), settled<D>(W8));
+  {
+    const int z = settled<D>(W8);
+    cd Z[D][D];
+    load_clf<D>(Z, clf, num, id + z, g.V);
+    mmac<D, true>(F, W8, Z);
+    load_clf<D>(Z, clf, num, om + z, g.V);
+    mmac<D, true>(F, Z, W8);
+  }
+#pragma unroll
+  for (int i = 0; i < D; i++)
+#pragma unroll
+    for (int j = 0; j < D; j++) F[i][j] = sign * F[i][j];
+  if (w > 0) {
+#pragma unroll
+    for (int e = 0; e < D * D; e++) ex[w - 1][e][lane] = make_double2(F[e / D][e % D].re, F[e / D][e % D].im);
+  }
+  __syncthreads();
+  if (w > 0 || k >= g.VH) return;
+#pragma unroll
+  for (int n = 0; n < 2; n++)
+#pragma unroll
+    for (int e = 0; e < D * D; e++) {
+      const double2 v = ex[n][e][lane];
+      F[e / D][e % D] = F[e / D][e % D] + cd(v.x, v.y);
+    }
+  L(W8, id, mu, false);
+  cd M[D][D];
+  mmac<D, false>(M, W8, F);
+  project_add<NG, D>(mom, mu, id, g.V, M, coeff, itr);
+}
+
 template <int D>
 struct FX {
   static constexpr int G = 64 / D;          // groups (x, mu) per wave
@@ -978,16 +1064,24 @@ __global__ void k_mom_to_ref(const double* __restrict__ src, double* __restrict_
   for (int a = 0; a < NG; a++) dst[(size_t)t * NG + a] = src[(size_t)(mu * NG + a) * V + id];
 }
 // clover force matrices -> reference cl_force layout [6*id + k] suNf
-__global__ void k_clf_to_ref(const double2* __restrict__ src, double* __restrict__ dst, int V, int D) {
+__global__ void k_clf_to_ref(const double* __restrict__ src, double* __restrict__ dst, int V, int D) {
   int t = blockIdx.x * 256 + threadIdx.x;
   if (t >= 6 * V) return;
   int id = t / 6, k = t % 6;
   double* o = dst + (size_t)t * 2 * D * D;
-  for (int e = 0; e < D * D; e++) {
-    double2 v = src[(size_t)(k * D * D + e) * V + id];
-    o[e] = v.x;
-    o[D * D + e] = v.y;
-  }
+  for (int i = 0; i < D; i++)
+    for (int j = 0; j < D; j++) {
+      double2 v;
+      if (D <= kClfPacked) {
+        const int hi = max(i, j), lo = min(i, j), e = hi == lo ? hi : D + hi * (hi - 1) + 2 * lo;
+        const double* q = src + (size_t)(k * D * D + e) * V + id;
+        v = i == j ? make_double2(0.0, q[0]) : make_double2(i > j ? q[0] : -q[0], q[V]);
+      } else {
+        v = ((const double2*)src)[(size_t)(k * D * D + i * D + j) * V + id];
+      }
+      o[i * D + j] = v.x;
+      o[D * D + i * D + j] = v.y;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -995,14 +1089,18 @@ __global__ void k_clf_to_ref(const double2* __restrict__ src, double* __restrict
 // ---------------------------------------------------------------------------
 static int ng_of(Ctx* c) { return c->nc * c->nc - 1; }
 
+static size_t clf_bytes(const Ctx* c) {
+  return (c->dr <= kClfPacked ? sizeof(double) : sizeof(double2)) * 6 * (size_t)c->dr * c->dr * c->g.V;
+}
+
 int force_alloc(Ctx* c) {
   if (!c->mom) {
     YH_HIP(hipMalloc(&c->mom, sizeof(double) * 4 * (size_t)ng_of(c) * c->g.V));
     YH_HIP(hipMemsetAsync(c->mom, 0, sizeof(double) * 4 * (size_t)ng_of(c) * c->g.V, c->stream));
   }
   if (!c->clf) {
-    YH_HIP(hipMalloc(&c->clf, sizeof(double2) * 6 * (size_t)c->dr * c->dr * c->g.V));
-    YH_HIP(hipMemsetAsync(c->clf, 0, sizeof(double2) * 6 * (size_t)c->dr * c->dr * c->g.V, c->stream));
+    YH_HIP(hipMalloc(&c->clf, clf_bytes(c)));
+    YH_HIP(hipMemsetAsync(c->clf, 0, clf_bytes(c), c->stream));
   }
   return YH_OK;
 }
@@ -1024,7 +1122,7 @@ int force_hop(Ctx* c, double coeff, const Field* lhs, const Field* rhs) {
   f.x[0] = lhs->half[0]; f.x[1] = lhs->half[1];
   f.y[0] = rhs->half[0]; f.y[1] = rhs->half[1];
   const double2* links = (const double2*)c->links[PREC_F64][RECON_18];
-  dim3 grid((4 * c->g.V + 255) / 256);
+  dim3 grid((c->g.VH + 63) / 64 * 2);
   YH_FORCE_MODELS(hipLaunchKernelGGL((k_force_hop<NG_, D_>), grid, dim3(256), 0, c->stream, f, links, c->mom, coeff, c->g, c->tab_itr));
   YH_HIP(hipGetLastError());
   return YH_OK;
@@ -1037,14 +1135,18 @@ int force_clover_site(Ctx* c, double residue, const Field* lhs, const Field* rhs
   f.x[0] = lhs->half[0]; f.x[1] = lhs->half[1];
   f.y[0] = rhs->half[0]; f.y[1] = rhs->half[1];
   dim3 grid((c->g.V + 255) / 256);
+#define YH_SITE(DD)                                                                                              \
+  hipLaunchKernelGGL((k_force_clover_site<DD, (DD <= kClfPacked)>), grid, dim3(256), 0, c->stream, f, (double*)c->clf, \
+                     residue, c->g)
   switch (c->dr) {
-    case 2: hipLaunchKernelGGL(k_force_clover_site<2>, grid, dim3(256), 0, c->stream, f, (double2*)c->clf, residue, c->g); break;
-    case 3: hipLaunchKernelGGL(k_force_clover_site<3>, grid, dim3(256), 0, c->stream, f, (double2*)c->clf, residue, c->g); break;
-    case 4: hipLaunchKernelGGL(k_force_clover_site<4>, grid, dim3(256), 0, c->stream, f, (double2*)c->clf, residue, c->g); break;
-    case 6: hipLaunchKernelGGL(k_force_clover_site<6>, grid, dim3(256), 0, c->stream, f, (double2*)c->clf, residue, c->g); break;
-    case 8: hipLaunchKernelGGL(k_force_clover_site<8>, grid, dim3(256), 0, c->stream, f, (double2*)c->clf, residue, c->g); break;
+    case 2: YH_SITE(2); break;
+    case 3: YH_SITE(3); break;
+    case 4: YH_SITE(4); break;
+    case 6: YH_SITE(6); break;
+    case 8: YH_SITE(8); break;
     default: set_error("unsupported representation dimension"); return YH_ERR_UNSUPPORTED;
   }
+#undef YH_SITE
   YH_HIP(hipGetLastError());
   return YH_OK;
 }
@@ -1056,11 +1158,11 @@ int force_logdet(Ctx* c, double mass, double coeff) {
   dim3 grid((c->g.VH + 127) / 128);
   const double2* inv = (const double2*)c->clinv[PREC_F64];
   switch (c->dr) {
-    case 2: hipLaunchKernelGGL(k_force_logdet<2>, grid, dim3(128), 0, c->stream, inv, (double2*)c->clf, coeff, c->g); break;
-    case 3: hipLaunchKernelGGL(k_force_logdet<3>, grid, dim3(128), 0, c->stream, inv, (double2*)c->clf, coeff, c->g); break;
-    case 4: hipLaunchKernelGGL(k_force_logdet<4>, grid, dim3(128), 0, c->stream, inv, (double2*)c->clf, coeff, c->g); break;
-    case 6: hipLaunchKernelGGL(k_force_logdet<6>, grid, dim3(128), 0, c->stream, inv, (double2*)c->clf, coeff, c->g); break;
-    case 8: hipLaunchKernelGGL(k_force_logdet<8>, grid, dim3(128), 0, c->stream, inv, (double2*)c->clf, coeff, c->g); break;
+    case 2: hipLaunchKernelGGL(k_force_logdet<2>, grid, dim3(128), 0, c->stream, inv, (double*)c->clf, coeff, c->g); break;
+    case 3: hipLaunchKernelGGL(k_force_logdet<3>, grid, dim3(128), 0, c->stream, inv, (double*)c->clf, coeff, c->g); break;
+    case 4: hipLaunchKernelGGL(k_force_logdet<4>, grid, dim3(128), 0, c->stream, inv, (double*)c->clf, coeff, c->g); break;
+    case 6: hipLaunchKernelGGL(k_force_logdet<6>, grid, dim3(128), 0, c->stream, inv, (double*)c->clf, coeff, c->g); break;
+    case 8: hipLaunchKernelGGL(k_force_logdet<8>, grid, dim3(128), 0, c->stream, inv, (double*)c->clf, coeff, c->g); break;
     default: set_error("unsupported representation dimension"); return YH_ERR_UNSUPPORTED;
   }
   YH_HIP(hipGetLastError());
@@ -1072,12 +1174,17 @@ int force_clover_core(Ctx* c, double dt) {
   if ((rc = force_alloc(c))) return rc;
   double coeff = c->csw * dt / 8.0;
   const double2* links = (const double2*)c->links[PREC_F64][RECON_18];
-  YH_FORCE_MODELS(const int groups = 64 / D_;
-                  const unsigned nsb = (unsigned)((c->g.V + groups - 1) / groups);
-                  dim3 grid = c->force_order < 0 ? dim3(nsb, 4) : dim3(4 * nsb);
-                  hipLaunchKernelGGL((k_force_clover_x<NG_, D_>), grid, dim3(64), 0, c->stream,
-                                     (const double2*)c->clf, links, c->mom, coeff, c->g, c->tab_itr,
-                                     c->force_order));
+  YH_FORCE_MODELS(
+      if constexpr (D_ <= kClfPacked) {
+        hipLaunchKernelGGL((k_force_clover_nu<NG_, D_>), dim3((c->g.VH + 63) / 64 * 8), dim3(192), 0, c->stream,
+                           (const double*)c->clf, links, c->mom, coeff, c->g, c->tab_itr);
+      } else {
+        const int groups = 64 / D_;
+        const unsigned nsb = (unsigned)((c->g.V + groups - 1) / groups);
+        dim3 grid = c->force_order < 0 ? dim3(nsb, 4) : dim3(4 * nsb);
+        hipLaunchKernelGGL((k_force_clover_x<NG_, D_>), grid, dim3(64), 0, c->stream, (const double2*)c->clf, links,
+                           c->mom, coeff, c->g, c->tab_itr, c->force_order);
+      });
   YH_HIP(hipGetLastError());
   return YH_OK;
 }
@@ -1105,7 +1212,7 @@ int zero_bc_half(Ctx* c, Field* f, int parity) {
 int clover_force_zero(Ctx* c) {
   int rc;
   if ((rc = force_alloc(c))) return rc;
-  YH_HIP(hipMemsetAsync(c->clf, 0, sizeof(double2) * 6 * (size_t)c->dr * c->dr * c->g.V, c->stream));
+  YH_HIP(hipMemsetAsync(c->clf, 0, clf_bytes(c), c->stream));
   return YH_OK;
 }
 
@@ -1144,7 +1251,7 @@ int clover_force_download(Ctx* c, double* host) {
   size_t n = (size_t)6 * c->g.V * 2 * c->dr * c->dr;
   double* d;
   YH_HIP(hipMalloc(&d, n * sizeof(double)));
-  hipLaunchKernelGGL(k_clf_to_ref, dim3((6 * c->g.V + 255) / 256), dim3(256), 0, c->stream, (const double2*)c->clf, d,
+  hipLaunchKernelGGL(k_clf_to_ref, dim3((6 * c->g.V + 255) / 256), dim3(256), 0, c->stream, (const double*)c->clf, d,
                      c->g.V, c->dr);
   hipError_t e = hipMemcpyAsync(host, d, n * sizeof(double), hipMemcpyDeviceToHost, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
