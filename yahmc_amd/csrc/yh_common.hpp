@@ -339,9 +339,10 @@ __device__ __forceinline__ R load_spinor_q(Cx<R> (&s)[4][D], const void* base, c
 }
 
 // NT: write with non-temporal stores (a field no later access of the same
-// kernel reads)
-template <int PREC, int D, typename R, bool NT = false>
-__device__ __forceinline__ void store_spinor(void* base, float* nrm, int site, int stride, const Cx<R> (&s)[4][D]) {
+// kernel reads).  SEEN (16-bit): s becomes the rounded field, as load_spinor
+// would return it
+template <int PREC, int D, typename R, bool NT = false, bool SEEN = false, typename S>
+__device__ __forceinline__ void store_spinor(void* base, float* nrm, int site, int stride, S&& s) {
   if constexpr (PREC == PREC_F64) {
     double2* p = (double2*)base;
 #pragma unroll
@@ -376,6 +377,10 @@ __device__ __forceinline__ void store_spinor(void* base, float* nrm, int site, i
       for (int q = 0; q < 4; q++) {
         int c = 4 * k + q;
         w[q] = pack_q2((float)s[c / D][c % D].re * inv, (float)s[c / D][c % D].im * inv);
+        if constexpr (SEEN) {
+          const float sc = mx * Q_UNIT;
+          s[c / D][c % D] = Cx<R>((R)(q2r_lo(w[q]) * sc), (R)(q2r_hi(w[q]) * sc));
+        }
       }
       const uint4 v = make_uint4(w[0], w[1], w[2], w[3]);
       if constexpr (NT) st_stream(&p[(size_t)k * stride + site], v);

@@ -522,22 +522,13 @@ __global__ void __launch_bounds__(YH_HOP_BLOCK, hop_min_waves<PREC>()) k_hop(Hop
           acc[3][i] = Cx<R>(-acc[3][i].re, -acc[3][i].im);
         }
       }
-      store_spinor<PREC, D, R, PREC == PREC_F64>(a.out, a.out_nrm, k, g.VHpad, acc);
+      // the norm is that of the stored (16-bit: rounded) field
+      store_spinor<PREC, D, R, PREC == PREC_F64, true>(a.out, a.out_nrm, k, g.VHpad, acc);
       if (a.reduce) {
-        if constexpr (PREC == PREC_F16) {
-          // reduce what was stored (the rounded field), as a consumer sees it
-          Cx<R> back[4][D];
-          load_spinor<PREC, D, R>(back, a.out, a.out_nrm, k, g.VHpad);
 #pragma unroll
-          for (int s = 0; s < 4; s++)
+        for (int s = 0; s < 4; s++)
 #pragma unroll
-            for (int i = 0; i < D; i++) nrm2 += (double)back[s][i].re * back[s][i].re + (double)back[s][i].im * back[s][i].im;
-        } else {
-#pragma unroll
-          for (int s = 0; s < 4; s++)
-#pragma unroll
-            for (int i = 0; i < D; i++) nrm2 += (double)acc[s][i].re * acc[s][i].re + (double)acc[s][i].im * acc[s][i].im;
-        }
+          for (int i = 0; i < D; i++) nrm2 += (double)acc[s][i].re * acc[s][i].re + (double)acc[s][i].im * acc[s][i].im;
       }
     }
   }

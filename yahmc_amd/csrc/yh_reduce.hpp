@@ -65,8 +65,19 @@ __device__ bool block_reduce_finish(double (&v)[NR], double* partials, int nblk,
   if (!is_last) return false;
 #pragma unroll
   for (int r = 0; r < NR; r++) {
+    // eight loads in flight at a time (added in order): each is a trip past
+    // the L2, and one by one they are the tail of every reduction
     double s = 0.0;
-    for (int i = threadIdx.x; i < nblk; i += NT) s += __hip_atomic_load(&partials[(size_t)r * nblk + i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i0 = threadIdx.x; i0 < nblk; i0 += 8 * NT) {
+      double t[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        const int i = i0 + u * NT;
+        t[u] = i < nblk ? __hip_atomic_load(&partials[(size_t)r * nblk + i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < 8; u++) s += t[u];
+    }
     s = wave_sum(s);
     __syncthreads();
     if (lane == 0) sm[r][w] = s;
