@@ -428,7 +428,9 @@ int yh_synchronize(yh_ctx* ctx);
  * kernels (D_R <= 3) copy the window of input spinors their y / z
  * neighbours come from into LDS once per workgroup and read those
  * neighbours there (when a (t, x) plane holds a multiple of 256 sites);
- * default 3: FP64 and FP32 */
+ * default 3: FP64 and FP32.  Setting it selects kernels of one thread per
+ * site at every size (by default small lattices, up to 32,768 sites a
+ * parity, put a site's eight directions on eight waves) */
 #define YH_TUNE_HOP_STAGE 8
 /* order in which the clover-force kernel's workgroups take their (site
  * block, mu) work: -1 = all sites of one mu after another; q >= 0 = the

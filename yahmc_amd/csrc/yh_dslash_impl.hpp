@@ -23,6 +23,7 @@
 //   CLOV     out = scale * sum + D_ee self [; gamma5] [; |out|^2]
 //                                                        (second half of Dphi)
 #pragma once
+#include <type_traits>
 #include "yh_internal.hpp"
 #include "yh_reduce.hpp"
 
@@ -540,6 +541,310 @@ __global__ void __launch_bounds__(YH_HOP_BLOCK, hop_min_waves<PREC>()) k_hop(Hop
   }
 }
 
+// ---------------------------------------------------------------------------
+// Small lattices: a site's eight directions on eight waves (D_R <= 6).  With
+// one thread per site a lattice of up to ~65,000 sites a half keeps at most
+// one wave per SIMD, and the launch lasts as long as one thread's chain of
+// eight neighbour loads and products.  Here a workgroup takes 64 sites and
+// wave w the direction w: it loads one neighbour and one link and leaves the
+// transported half spinor in LDS; waves 0 and 1, which (D_R <= 4,
+// FP32 and 16-bit) have their chiral block of the clover term in flight
+// meanwhile, add the eight in the order of k_hop and finish spins 0, 1 and 2, 3.  FP64 and
+// FP32 results equal k_hop's bit for bit (FP64 norms are summed in another
+// order); 16-bit ones differ by the rounding of one multiplication.
+// Not for a call with a side output (aux), which keeps k_hop.
+template <int D, typename R>
+struct SplitArgs {
+  const HopArgs& a;
+  Cx<R> (*part)[2 * D][64];
+  int lane;
+};
+
+template <int W, int D, int PREC, int RECON, typename R>
+__device__ __forceinline__ void split_dir(const SplitArgs<D, R>& s, const int (&c)[4], int k) {
+  constexpr int MU = W >> 1;
+  constexpr bool FWD = !(W & 1);
+  typedef Proj<MU, FWD> P;
+  const HopArgs& a = s.a;
+  const Geom& g = a.g;
+  int n[4] = {c[0], c[1], c[2], c[3]};
+  n[MU] = FWD ? (c[MU] + 1 == g.L[MU] ? 0 : c[MU] + 1) : (c[MU] == 0 ? g.L[MU] - 1 : c[MU] - 1);
+  const int nidx = half_index(n[0], n[1], n[2], n[3], g), lidx = FWD ? k : nidx;
+  const bool flip = MU == 0 && g.bc == BC_ANTIPERIODIC && (FWD ? c[0] : n[0]) == 0;
+  typedef typename LinkStore<PREC, RECON, D>::vec LV;
+  const LV* lbase = (const LV*)(FWD ? a.lf : a.lb) + (size_t)MU * link_planes<PREC, RECON, D>() * g.VHpad;
+  Cx<R> x[4][D], u[D][D];
+  R sc = (R)1;
+  if constexpr (PREC == PREC_F16) sc = load_spinor_q<D, R>(x, a.in, a.in_nrm, nidx, g.VHpad) * (R)Q_UNIT;
+  else load_spinor<PREC, D, R>(x, a.in, a.in_nrm, nidx, g.VHpad);
+  load_link<PREC, RECON, D, R, false, PREC == PREC_F16>(u, lbase, lidx, g.VHpad);
+  if (flip) sc = -sc;
+  Cx<R> h[2][D];
+#pragma unroll
+  for (int i = 0; i < D; i++) {
+    h[0][i] = x[2][i] + unit_mul<P::PC0>(x[P::PI0][i]);
+    h[1][i] = x[3][i] + unit_mul<P::PC1>(x[P::PI1][i]);
+  }
+#pragma unroll
+  for (int i = 0; i < D; i++)
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      Cx<R> r((R)0, (R)0);
+#pragma unroll
+      for (int j = 0; j < D; j++) {
+        if constexpr (FWD) cmac(r, u[i][j], h[q][j]);
+        else cmac_conj(r, u[j][i], h[q][j]);
+      }
+      s.part[W][q * D + i][s.lane] = sc * r;
+    }
+}
+
+// acc[2 D] of chiral block B: += direction W's part
+template <int W, int B, int D, typename R>
+__device__ __forceinline__ void split_add(Cx<R> (&acc)[2 * D], const Cx<R> (*part)[2 * D][64], int lane) {
+  typedef Proj<(W >> 1), !(W & 1)> P;
+#pragma unroll
+  for (int i = 0; i < D; i++) {
+    if constexpr (B == 1) {
+      acc[i] = acc[i] + part[W][i][lane];
+      acc[D + i] = acc[D + i] + part[W][D + i][lane];
+    } else {
+      acc[i] = acc[i] + unit_mul<P::RC0>(part[W][P::RI0 * D + i][lane]);
+      acc[D + i] = acc[D + i] + unit_mul<P::RC1>(part[W][P::RI1 * D + i][lane]);
+    }
+  }
+}
+
+// components of chiral block B (2 D of them, spin-major) of a stored spinor
+template <int PREC, int D, int B, typename R>
+__device__ __forceinline__ void load_half_spinor(Cx<R> (&x)[2 * D], const void* base, const float* nrm, int site,
+                                                 int stride) {
+  constexpr int C0 = 2 * B * D;
+  if constexpr (PREC == PREC_F64) {
+    const double2* p = (const double2*)base;
+#pragma unroll
+    for (int i = 0; i < 2 * D; i++) {
+      const double2 v = p[(size_t)(C0 + i) * stride + site];
+      x[i] = Cx<R>((R)v.x, (R)v.y);
+    }
+  } else if constexpr (PREC == PREC_F32) {
+    const float4* p = (const float4*)base;
+#pragma unroll
+    for (int i = 0; i < D; i++) {
+      const float4 v = p[(size_t)(C0 / 2 + i) * stride + site];
+      x[2 * i] = Cx<R>((R)v.x, (R)v.y);
+      x[2 * i + 1] = Cx<R>((R)v.z, (R)v.w);
+    }
+  } else {
+    const uint4* p = (const uint4*)base;
+    const float sc = nrm[site] * Q_UNIT;
+#pragma unroll
+    for (int v = C0 / 4; v <= (C0 + 2 * D - 1) / 4; v++) {
+      const uint4 q = p[(size_t)v * stride + site];
+      const unsigned w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int i = 4 * v + e - C0;
+        if (i >= 0 && i < 2 * D) x[i] = Cx<R>((R)(q2r_lo(w[e]) * sc), (R)(q2r_hi(w[e]) * sc));
+      }
+    }
+  }
+}
+
+template <int D, int PREC, int RECON, int EPI>
+__global__ void __launch_bounds__(512) k_hop_split(HopArgs a) {
+  typedef typename SpinorStore<PREC, D>::real R;
+  constexpr int N = 2 * D;
+  if (a.skip && *a.skip) return;
+  __shared__ Cx<R> part[8][N][64];
+  __shared__ float xmax[2][64];      // 16-bit: largest component of each block
+  __shared__ Cx<float> xcomp[2][64];  // 16-bit, odd D_R: the last two components of block 0
+  const Geom& g = a.g;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int k = blockIdx.x * 64 + lane;
+  const bool on = k < g.VH;
+  const int kk = on ? k : g.VH - 1;  // lanes past the end compute on the last site and write nothing
+  int c[4];
+  site_coords(kk, a.parity, g, c);
+  const SplitArgs<D, R> s{a, part, lane};
+  // the clover block and own spinor of waves 0 and 1, in flight during the hop;
+  // LATE: read where they are used (STREAM: a few entries at a time), since
+  // they would spill beside the sums
+  constexpr bool STREAM = PREC == PREC_F64 && D >= 4, LATE = (PREC == PREC_F64 && D >= 4) || D >= 6;
+  R cl[LATE ? 1 : N * N];
+  Cx<R> xs[N];
+  auto pre = [&](auto bc) {
+    constexpr int B = bc();
+    if constexpr (EPI != EPI_PLAIN && !LATE) load_clover_block<PREC, D, R>(cl, a.clov, B, kk, g.VHpad, a.clov_nrm);
+    if constexpr (EPI == EPI_CLOV && !LATE) load_half_spinor<PREC, D, B, R>(xs, a.self, a.self_nrm, kk, g.VHpad);
+  };
+  switch (w) {
+    case 0: split_dir<0, D, PREC, RECON, R>(s, c, kk); pre(std::integral_constant<int, 0>()); break;
+    case 1: split_dir<1, D, PREC, RECON, R>(s, c, kk); pre(std::integral_constant<int, 1>()); break;
+    case 2: split_dir<2, D, PREC, RECON, R>(s, c, kk); break;
+    case 3: split_dir<3, D, PREC, RECON, R>(s, c, kk); break;
+    case 4: split_dir<4, D, PREC, RECON, R>(s, c, kk); break;
+    case 5: split_dir<5, D, PREC, RECON, R>(s, c, kk); break;
+    case 6: split_dir<6, D, PREC, RECON, R>(s, c, kk); break;
+    default: split_dir<7, D, PREC, RECON, R>(s, c, kk); break;
+  }
+  __syncthreads();
+  double nrm2 = 0.0;
+  Cx<R> o[N];
+  float mx = 0.f;
+  auto finish = [&](auto bc) {
+    constexpr int B = bc();
+    Cx<R> acc[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) acc[i] = Cx<R>((R)0, (R)0);
+    // FP64 and D_R = 6: two directions' parts in registers at a time (opaque zero)
+    int l = lane;
+    auto pace = [&]() {
+      if constexpr (PREC == PREC_F64 || D >= 6) {
+#pragma unroll
+        for (int i = 0; i < N; i++) __asm__ volatile("" : "+v"(acc[i].re), "+v"(acc[i].im));
+        int z;
+        __asm__ volatile("v_mov_b32 %0, 0" : "=v"(z));
+        l = lane + z;
+      }
+    };
+    split_add<0, B, D, R>(acc, part, l);
+    split_add<1, B, D, R>(acc, part, l);
+    pace();
+    split_add<2, B, D, R>(acc, part, l);
+    split_add<3, B, D, R>(acc, part, l);
+    pace();
+    split_add<4, B, D, R>(acc, part, l);
+    split_add<5, B, D, R>(acc, part, l);
+    pace();
+    split_add<6, B, D, R>(acc, part, l);
+    split_add<7, B, D, R>(acc, part, l);
+    pace();
+    const bool bz = bc_zero_slice(c[0], g);
+    const R scale = bz ? (R)0 : (R)a.scale;
+#pragma unroll
+    for (int i = 0; i < N; i++) acc[i] = scale * acc[i];
+    if constexpr (EPI == EPI_PLAIN) {
+#pragma unroll
+      for (int i = 0; i < N; i++) o[i] = acc[i];
+    } else {
+      if constexpr (EPI == EPI_CLOV) {
+        if constexpr (LATE) load_half_spinor<PREC, D, B, R>(xs, a.self, a.self_nrm, kk + l - lane, g.VHpad);
+        const bool zs = a.zero_self_bc && bz;
+#pragma unroll
+        for (int i = 0; i < N; i++) xs[i] = zs ? Cx<R>((R)0, (R)0) : xs[i];
+      } else {
+#pragma unroll
+        for (int i = 0; i < N; i++) xs[i] = acc[i];
+      }
+      if constexpr (STREAM) herm_mv_f64_stream<N>(o, a.clov, B, kk + l - lane, g.VHpad, xs);
+      else if constexpr (LATE) {
+        R cb[N * N];
+        load_clover_block<PREC, D, R>(cb, a.clov, B, kk + l - lane, g.VHpad, a.clov_nrm);
+        herm_mv<N, R>(o, cb, xs);
+      } else herm_mv<N, R>(o, cl, xs);
+      if constexpr (EPI == EPI_CLOV) {
+        const R dg = (R)(a.diag + bc_cf_shift(c[0], g));
+#pragma unroll
+        for (int i = 0; i < N; i++) o[i] = acc[i] + o[i] + dg * xs[i];
+        if (B == 1 && a.gamma5) {
+#pragma unroll
+          for (int i = 0; i < N; i++) o[i] = Cx<R>(-o[i].re, -o[i].im);
+        }
+      }
+    }
+    constexpr int C0 = B * N;
+    if constexpr (PREC == PREC_F64) {
+      double2* p = (double2*)a.out;
+      if (on) {
+#pragma unroll
+        for (int i = 0; i < N; i++) p[(size_t)(C0 + i) * g.VHpad + k] = make_double2(o[i].re, o[i].im);
+      }
+    } else if constexpr (PREC == PREC_F32) {
+      float4* p = (float4*)a.out;
+      if (on) {
+#pragma unroll
+        for (int i = 0; i < D; i++)
+          p[(size_t)(C0 / 2 + i) * g.VHpad + k] =
+              make_float4((float)o[2 * i].re, (float)o[2 * i].im, (float)o[2 * i + 1].re, (float)o[2 * i + 1].im);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < N; i++) mx = fmaxf(mx, fmaxf(fabsf((float)o[i].re), fabsf((float)o[i].im)));
+      xmax[B][lane] = mx;
+      if constexpr (B == 0 && D % 2 == 1) {
+        xcomp[0][lane] = Cx<float>((float)o[N - 2].re, (float)o[N - 2].im);
+        xcomp[1][lane] = Cx<float>((float)o[N - 1].re, (float)o[N - 1].im);
+      }
+    }
+  };
+  if (w == 0) finish(std::integral_constant<int, 0>());
+  else if (w == 1) finish(std::integral_constant<int, 1>());
+  if constexpr (PREC == PREC_F16) {
+    // the site's scale is the larger of the blocks' maxima; an odd D_R has one
+    // 16-byte vector that straddles the blocks, written by wave 1
+    __syncthreads();
+    auto store = [&](auto bc) {
+      constexpr int B = bc();
+      const float m = fmaxf(xmax[0][lane], xmax[1][lane]);
+      const float inv = m > 0.f ? 1.0f / m : 0.f, sc = m * Q_UNIT;
+      unsigned q[N];
+#pragma unroll
+      for (int i = 0; i < N; i++) {
+        q[i] = pack_q2((float)o[i].re * inv, (float)o[i].im * inv);
+        o[i] = Cx<R>((R)(q2r_lo(q[i]) * sc), (R)(q2r_hi(q[i]) * sc));  // as stored, for the norm
+      }
+      if (!on) return;
+      uint4* p = (uint4*)a.out;
+      if constexpr (D % 2 == 0) {
+#pragma unroll
+        for (int v = 0; v < D / 2; v++)
+          p[(size_t)(B * D / 2 + v) * g.VHpad + k] = make_uint4(q[4 * v], q[4 * v + 1], q[4 * v + 2], q[4 * v + 3]);
+      } else if constexpr (B == 0) {
+#pragma unroll
+        for (int v = 0; v < (D - 1) / 2; v++)
+          p[(size_t)v * g.VHpad + k] = make_uint4(q[4 * v], q[4 * v + 1], q[4 * v + 2], q[4 * v + 3]);
+      } else {
+        const Cx<float> e = xcomp[0][lane], f = xcomp[1][lane];
+        p[(size_t)((D - 1) / 2) * g.VHpad + k] =
+            make_uint4(pack_q2(e.re * inv, e.im * inv), pack_q2(f.re * inv, f.im * inv), q[0], q[1]);
+#pragma unroll
+        for (int v = 0; v < (D - 1) / 2; v++)
+          p[(size_t)((D + 1) / 2 + v) * g.VHpad + k] =
+              make_uint4(q[4 * v + 2], q[4 * v + 3], q[4 * v + 4], q[4 * v + 5]);
+      }
+      if constexpr (B == 0) a.out_nrm[k] = m;
+    };
+    if (w == 0) store(std::integral_constant<int, 0>());
+    else if (w == 1) store(std::integral_constant<int, 1>());
+  }
+  if constexpr (EPI == EPI_CLOV) {
+    if (a.reduce) {
+      if (w < 2 && on) {
+#pragma unroll
+        for (int i = 0; i < N; i++) nrm2 += (double)o[i].re * o[i].re + (double)o[i].im * o[i].im;
+      }
+      double v[1] = {nrm2};
+      block_reduce_finish<1, 512>(v, a.partials, gridDim.x, blockIdx.x, a.ticket, a.red_out);
+    }
+  }
+}
+
+// largest half volume that k_hop_split takes: two workgroups (64 sites each)
+// per CU.  H^2 through yh_Hphi_sq (three of its four hops split, ~10 us of it
+// the call), split / one thread per site, in us:
+//                   VH 4,096       14,400        32,768        49,152
+//   SU(3) FP64    41.1 /  67.3  51.2 /  81.3  76.8 /  84.1  105.6 /  95.2
+//   SU(3) 16-bit  30.9 /  39.8  32.9 /  42.5  43.5 /  44.0   51.8 /  46.0
+//   SU(4) FP32    39.6 /  54.8  49.2 /  73.0  71.4 /  78.6   96.7 /  88.0
+//   sextet FP64   83.3 / 177.5  114.3 / 195.0  212.2 / 214.3  324.3 / 277.8
+//   SU(2) FP32    28.1 /  34.6  30.2 /  35.9  35.6 /  37.1   44.2 /  40.2
+// D_R = 8 keeps one thread per site (0).
+template <int D>
+constexpr int split_limit() {
+  return D <= 6 ? 32768 : 0;
+}
+
 // standalone clover apply (Dphi_ee / Dphi_oo) and inverse (Dphi_oo_inv)
 // (library/dirac.cpp:25-225)
 template <int D, int PREC, bool INV>
@@ -764,6 +1069,18 @@ int hop_mr_dispatch_d(Ctx* c, const HopArgsM& m, int prec, int nr, int epi) {
 template <int D, int PREC, int RECON>
 static int hop_dispatch_epi(Ctx* c, const HopArgs& a, int epi, hipStream_t st) {
   dim3 grid((c->g.VH + YH_HOP_BLOCK - 1) / YH_HOP_BLOCK), block(YH_HOP_BLOCK);
+  if constexpr (split_limit<D>() > 0) {
+    if (c->hop_split && !a.aux && c->g.VH <= split_limit<D>()) {
+      const dim3 sgrid((c->g.VH + 63) / 64);
+      switch (epi) {
+        case EPI_PLAIN: hipLaunchKernelGGL((k_hop_split<D, PREC, RECON, EPI_PLAIN>), sgrid, dim3(512), 0, st, a); break;
+        case EPI_CLOVINV: hipLaunchKernelGGL((k_hop_split<D, PREC, RECON, EPI_CLOVINV>), sgrid, dim3(512), 0, st, a); break;
+        default: hipLaunchKernelGGL((k_hop_split<D, PREC, RECON, EPI_CLOV>), sgrid, dim3(512), 0, st, a); break;
+      }
+      YH_HIP(hipGetLastError());
+      return YH_OK;
+    }
+  }
   if constexpr (D <= 3) {
     // LDS-staged y / z neighbours (yh_tune YH_TUNE_HOP_STAGE) where the
     // geometry allows it (Stage::usable; the kernel has a barrier)

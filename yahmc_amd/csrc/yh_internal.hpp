@@ -104,6 +104,8 @@ struct Ctx {
   // hop kernels (D_R <= 3) of the precisions in this mask (bit = precision)
   // read y / z neighbours from an LDS-staged window
   int hop_stage = (1 << PREC_F64) | (1 << PREC_F32);
+  // small lattices run a site's directions on eight waves (k_hop_split)
+  int hop_split = 1;
   int force_order = 0;  // YH_TUNE_FORCE_ORDER
   // solver chunks are captured once into a HIP graph and replayed
   int use_graphs = 1;
