@@ -3,15 +3,22 @@
 //
 // Per iteration and right-hand side: H^2 p (four fused hop kernels, the last
 // one also reducing <p, H^2 p> = |H p|^2), then two fused update kernels:
-//   k_ms_x : r += beta q ; |r|^2 -> alpha; the last workgroup computes the
-//            zeta coefficients c3_s, the solution step bt_s = beta c3_s / c2_s
-//            and the direction factor of every active shift and the
+//   k_ms_x : r_new = r + beta q ; |r|^2 -> alpha; the last workgroup computes
+//            the zeta coefficients c3_s, the solution step bt_s = beta c3_s /
+//            c2_s and the direction factor of every active shift and the
 //            convergence flags
-//   k_ms_k : for the shifts that were active in this iteration, in one pass
-//            over x_s and k_s:  x_s -= bt_s k_s ;  k_s = at_s k_s + c3_s r
+//   k_ms_p : p = alpha p + r
+// and every MS_RING iterations
+//   k_ms_k : for each of those iterations in turn, for the shifts that were
+//            active in it:  x_s -= bt_s k_s ;  k_s = at_s k_s + c3_s r
 //            (the solution step uses k_s before its update, as the
-//            reference's order x_s -= bt k_s, then k_s = ... has it) ;
-//            p = alpha p + r
+//            reference's order x_s -= bt k_s, then k_s = ... has it).
+// x_s and k_s take no part in the recurrence of r and p, so their updates
+// wait until MS_RING residuals are there and go through memory once for all:
+// the shift vectors, 4 of the ~4.5 field passes per shift and iteration, move
+// a quarter of the bytes, by the same operations in the same order (results
+// are unchanged bit for bit).  24^3 x 48 SU(2) adjoint, 12 shifts: 363 us an
+// iteration when each updated them (6.5 TB/s), 121 + 27 for k_ms_k / 4 + k_ms_p.
 // The host only queues chunks of iterations and reads one flag per chunk.
 // Right-hand sides are independent recurrences sharing the gauge field; they
 // are interleaved iteration by iteration so consecutive hop launches reuse
@@ -23,13 +30,15 @@
 
 namespace yh {
 
-enum { MS_MAX = 48 };
+enum { MS_MAX = 48, MS_RING = 4 };
 
 struct MsState {
   double rr, pap, beta, beta_old, alpha, norm, target;
   int done, iters, nshift, notconv;
-  double shift[MS_MAX], c1[MS_MAX], c2[MS_MAX], c3[MS_MAX], at[MS_MAX], bt[MS_MAX];
-  int act[MS_MAX], upd[MS_MAX];
+  double shift[MS_MAX], c1[MS_MAX], c2[MS_MAX];
+  // coefficients of the iterations whose x_s, k_s updates are pending
+  double c3[MS_RING][MS_MAX], at[MS_RING][MS_MAX], bt[MS_RING][MS_MAX];
+  int act[MS_MAX], upd[MS_RING][MS_MAX];
 };
 
 struct MsFields {
@@ -38,9 +47,8 @@ struct MsFields {
 };
 
 template <int D>
-__global__ void __launch_bounds__(256) k_ms_x(MsState* st, const MsFields* __restrict__ mf, void* r, const void* q,
+__global__ void __launch_bounds__(256) k_ms_x(MsState* st, int slot, const void* r, void* rnew, const void* q,
                                               double* partials, unsigned* ticket, Geom g) {
-  (void)mf;
   if (st->done) return;
   const double atmp = st->rr, btmp = st->pap;
   const double beta_old = st->beta;
@@ -60,7 +68,7 @@ __global__ void __launch_bounds__(256) k_ms_x(MsState* st, const MsFields* __res
         R[a][i] = Cx<double>(R[a][i].re + beta * Q[a][i].re, R[a][i].im + beta * Q[a][i].im);
         v[0] += R[a][i].re * R[a][i].re + R[a][i].im * R[a][i].im;
       }
-    store_spinor<PREC_F64, D, double>(r, nullptr, k, g.VHpad, R);
+    store_spinor<PREC_F64, D, double>(rnew, nullptr, k, g.VHpad, R);
   }
   double res[1];
   if (block_reduce_finish<1, 256>(v, partials, gridDim.x, blockIdx.x, ticket, res) && threadIdx.x == 0) {
@@ -68,13 +76,13 @@ __global__ void __launch_bounds__(256) k_ms_x(MsState* st, const MsFields* __res
     const double alpha_new = rr_new / atmp;
     int notconv = 0;
     for (int s = 0; s < ns; s++) {
-      st->upd[s] = st->act[s];
+      st->upd[slot][s] = st->act[s];
       if (!st->act[s]) continue;
       double c1 = st->c1[s], c2 = st->c2[s];
       double c3 = c2 * c1 * beta_old / (beta * alpha * (c1 - c2) + c1 * beta_old * (1 - st->shift[s] * beta));
-      st->bt[s] = beta * (c3 / c2);
-      st->c3[s] = c3;
-      st->at[s] = alpha_new * (c3 * c3) / (c2 * c2);
+      st->bt[slot][s] = beta * (c3 / c2);
+      st->c3[slot][s] = c3;
+      st->at[slot][s] = alpha_new * (c3 * c3) / (c2 * c2);
       if (rr_new * c3 * c3 < st->target) st->act[s] = 0;
       else notconv++;
       st->c1[s] = c2;
@@ -90,98 +98,102 @@ __global__ void __launch_bounds__(256) k_ms_x(MsState* st, const MsFields* __res
   }
 }
 
-template <int D>
-__global__ void __launch_bounds__(256) k_ms_k(MsState* st, const MsFields* __restrict__ mf, const void* r, void* p,
-                                              unsigned* ticket, Geom g) {
-  // a chunk can run past the final iteration: then no shift is marked for
-  // update (cleared below) and p is left alone
-  const int ns = st->nshift;
-  const bool move_p = !st->done;
+// p = alpha p + r (one component plane per blockIdx.y)
+__global__ void __launch_bounds__(256) k_ms_p(const MsState* st, const double2* __restrict__ r,
+                                              double2* __restrict__ p, Geom g) {
+  if (st->done) return;
   const int k = blockIdx.x * 256 + threadIdx.x;
+  if (k >= g.VH) return;
+  const double alpha = st->alpha;
+  const size_t o = (size_t)blockIdx.y * g.VHpad + k;
+  const double2 a = r[o], b = p[o];
+  p[o] = make_double2(alpha * b.x + a.x, alpha * b.y + a.y);
+}
+
+struct MsRing {
+  const double2* r[MS_RING];  // residuals of the pending iterations
+};
+
+// the pending x_s, k_s updates (one component plane per blockIdx.y), four
+// shifts' vectors in flight at a time
+__global__ void __launch_bounds__(256) k_ms_k(const MsState* st, const MsFields* __restrict__ mf, MsRing ring,
+                                              Geom g) {
+  const int ns = st->nshift;
+  const int k = blockIdx.x * 256 + threadIdx.x;
+  // a shift active in a later iteration of the ring was active in the first
+  int marks = 0;
+  for (int s = 0; s < ns; s++) marks |= st->upd[0][s];
+  if (!marks) return;
   if (k < g.VH) {
-    Cx<double> R[4][D];
-    load_spinor<PREC_F64, D, double>(R, r, nullptr, k, g.VHpad);
-    for (int s = 0; s < ns; s++) {
-      if (!st->upd[s]) continue;
-      const double at = st->at[s], c3 = st->c3[s], bt = st->bt[s];
-      Cx<double> K[4][D], X[4][D];
-      load_spinor<PREC_F64, D, double>(K, mf->k[s], nullptr, k, g.VHpad);
-      load_spinor<PREC_F64, D, double>(X, mf->x[s], nullptr, k, g.VHpad);
+    const size_t o = (size_t)blockIdx.y * g.VHpad + k;
+    double2 R[MS_RING];
 #pragma unroll
-      for (int a = 0; a < 4; a++)
+    for (int j = 0; j < MS_RING; j++) R[j] = ring.r[j][o];
+    constexpr int G = 4;
+    for (int s0 = 0; s0 < ns; s0 += G) {
+      double2 X[G], K[G];
 #pragma unroll
-        for (int i = 0; i < D; i++) {
-          X[a][i] = Cx<double>(X[a][i].re - bt * K[a][i].re, X[a][i].im - bt * K[a][i].im);
-          K[a][i] = Cx<double>(at * K[a][i].re + c3 * R[a][i].re, at * K[a][i].im + c3 * R[a][i].im);
+      for (int u = 0; u < G; u++) {
+        const int s = min(s0 + u, ns - 1);
+        X[u] = ((const double2*)mf->x[s])[o];
+        K[u] = ((const double2*)mf->k[s])[o];
+      }
+#pragma unroll
+      for (int u = 0; u < G; u++) {
+        const int s = s0 + u;
+        if (s >= ns || !st->upd[0][s]) continue;
+#pragma unroll
+        for (int j = 0; j < MS_RING; j++) {
+          if (!st->upd[j][s]) continue;
+          const double at = st->at[j][s], c3 = st->c3[j][s], bt = st->bt[j][s];
+          X[u] = make_double2(X[u].x - bt * K[u].x, X[u].y - bt * K[u].y);
+          K[u] = make_double2(at * K[u].x + c3 * R[j].x, at * K[u].y + c3 * R[j].y);
         }
-      store_spinor<PREC_F64, D, double>(mf->x[s], nullptr, k, g.VHpad, X);
-      store_spinor<PREC_F64, D, double>(mf->k[s], nullptr, k, g.VHpad, K);
+        ((double2*)mf->x[s])[o] = X[u];
+        ((double2*)mf->k[s])[o] = K[u];
+      }
     }
-    if (move_p) {
-      const double alpha = st->alpha;
-      Cx<double> P[4][D];
-      load_spinor<PREC_F64, D, double>(P, p, nullptr, k, g.VHpad);
-#pragma unroll
-      for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int i = 0; i < D; i++) P[a][i] = Cx<double>(alpha * P[a][i].re + R[a][i].re, alpha * P[a][i].im + R[a][i].im);
-      store_spinor<PREC_F64, D, double>(p, nullptr, k, g.VHpad, P);
-    }
-  }
-  // last workgroup: clear the update marks once every workgroup has used them
-  // (every wave of this workgroup has read the marks before the barrier;
-  // the ticket is a relaxed agent-scope atomic, as in block_reduce_finish)
-  __shared__ int last;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    stores_complete();
-    unsigned t = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    last = (t == gridDim.x - 1);
-  }
-  __syncthreads();
-  if (last && threadIdx.x == 0) {
-    for (int s = 0; s < ns; s++) st->upd[s] = 0;
-    __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
+
+// no update is pending any more (a kernel of its own: the grid of k_ms_k has
+// tens of thousands of workgroups, and a ticket for each would serialise)
+__global__ void __launch_bounds__(MS_RING * MS_MAX) k_ms_clear(MsState* st) { (&st->upd[0][0])[threadIdx.x] = 0; }
 
 // ---------------------------------------------------------------------------
 template <int D>
-static int launch_x(Ctx* c, MsState* st, const MsFields* mf, Field* r, const Field* q) {
+static int launch_x(Ctx* c, MsState* st, int slot, const Field* r, Field* rnew, const Field* q) {
   dim3 grid((c->g.VH + 255) / 256);
-  hipLaunchKernelGGL(k_ms_x<D>, grid, dim3(256), 0, c->stream, st, mf, r->half[0], q->half[0], c->partials, c->ticket,
-                     c->g);
+  hipLaunchKernelGGL(k_ms_x<D>, grid, dim3(256), 0, c->stream, st, slot, r->half[0], rnew->half[0], q->half[0],
+                     c->partials, c->ticket, c->g);
   YH_HIP(hipGetLastError());
   return YH_OK;
 }
 
-template <int D>
-static int launch_k(Ctx* c, MsState* st, const MsFields* mf, const Field* r, Field* p) {
-  dim3 grid((c->g.VH + 255) / 256);
-  hipLaunchKernelGGL(k_ms_k<D>, grid, dim3(256), 0, c->stream, st, mf, r->half[0], p->half[0], c->ticket, c->g);
+static int ms_p(Ctx* c, const MsState* st, const Field* r, Field* p) {
+  dim3 grid((c->g.VH + 255) / 256, 4 * c->dr);
+  hipLaunchKernelGGL(k_ms_p, grid, dim3(256), 0, c->stream, st, (const double2*)r->half[0], (double2*)p->half[0], c->g);
   YH_HIP(hipGetLastError());
   return YH_OK;
 }
 
-static int ms_x(Ctx* c, MsState* st, const MsFields* mf, Field* r, const Field* q) {
-  switch (c->dr) {
-    case 2: return launch_x<2>(c, st, mf, r, q);
-    case 3: return launch_x<3>(c, st, mf, r, q);
-    case 4: return launch_x<4>(c, st, mf, r, q);
-    case 6: return launch_x<6>(c, st, mf, r, q);
-    case 8: return launch_x<8>(c, st, mf, r, q);
-  }
-  set_error("unsupported representation dimension");
-  return YH_ERR_UNSUPPORTED;
+static int ms_k(Ctx* c, MsState* st, const MsFields* mf, Field* const* ring) {
+  MsRing R;
+  for (int j = 0; j < MS_RING; j++) R.r[j] = (const double2*)ring[j]->half[0];
+  dim3 grid((c->g.VH + 255) / 256, 4 * c->dr);
+  hipLaunchKernelGGL(k_ms_k, grid, dim3(256), 0, c->stream, st, mf, R, c->g);
+  hipLaunchKernelGGL(k_ms_clear, dim3(1), dim3(MS_RING * MS_MAX), 0, c->stream, st);
+  YH_HIP(hipGetLastError());
+  return YH_OK;
 }
 
-static int ms_k(Ctx* c, MsState* st, const MsFields* mf, const Field* r, Field* p) {
+static int ms_x(Ctx* c, MsState* st, int slot, const Field* r, Field* rnew, const Field* q) {
   switch (c->dr) {
-    case 2: return launch_k<2>(c, st, mf, r, p);
-    case 3: return launch_k<3>(c, st, mf, r, p);
-    case 4: return launch_k<4>(c, st, mf, r, p);
-    case 6: return launch_k<6>(c, st, mf, r, p);
-    case 8: return launch_k<8>(c, st, mf, r, p);
+    case 2: return launch_x<2>(c, st, slot, r, rnew, q);
+    case 3: return launch_x<3>(c, st, slot, r, rnew, q);
+    case 4: return launch_x<4>(c, st, slot, r, rnew, q);
+    case 6: return launch_x<6>(c, st, slot, r, rnew, q);
+    case 8: return launch_x<8>(c, st, slot, r, rnew, q);
   }
   set_error("unsupported representation dimension");
   return YH_ERR_UNSUPPORTED;
@@ -195,7 +207,8 @@ int mshift_device(Ctx* c, const yh_inv_par* par, int nrhs, int num, const double
   int rc = YH_OK;
   const int recon = default_recon(c, PREC_F64);
   struct Rhs {
-    Field *r, *p, *q;
+    Field* r[MS_RING];  // residual of iteration i of a chunk in r[i % MS_RING]
+    Field *p, *q;
     Field *t1 = nullptr, *t2 = nullptr;  // operator temporaries of the multi-RHS path
     std::vector<Field*> k;
   };
@@ -224,13 +237,14 @@ int mshift_device(Ctx* c, const yh_inv_par* par, int nrhs, int num, const double
   std::vector<MsFields> hf(nrhs);
   for (int j = 0; j < nrhs && !rc; j++) {
     Rhs& R = rh[j];
-    if ((rc = alloc(&R.r)) || (rc = alloc(&R.p)) || (rc = alloc(&R.q))) break;
+    for (int i = 0; i < MS_RING && !rc; i++) rc = alloc(&R.r[i]);
+    if (rc || (rc = alloc(&R.p)) || (rc = alloc(&R.q))) break;
     if (batched && ((rc = alloc(&R.t1)) || (rc = alloc(&R.t2)))) break;
     R.k.resize(num);
     for (int s = 0; s < num && !rc; s++) rc = alloc(&R.k[s]);
     if (rc) break;
     // r = b ; p = b ; x_s = 0 ; k_s = b  (cg.cpp:35-43)
-    if ((rc = blas_copy(c, R.r, b[j], 0)) || (rc = blas_copy(c, R.p, b[j], 0))) break;
+    if ((rc = blas_copy(c, R.r[MS_RING - 1], b[j], 0)) || (rc = blas_copy(c, R.p, b[j], 0))) break;
     for (int s = 0; s < num && !rc; s++) {
       if ((rc = field_zero(c, x[j * num + s], YH_BOTH))) break;
       rc = blas_copy(c, R.k[s], b[j], 0);
@@ -261,6 +275,7 @@ int mshift_device(Ctx* c, const yh_inv_par* par, int nrhs, int num, const double
     if (he != hipSuccess) { set_error(hipGetErrorString(he)); rc = YH_ERR_HIP; }
   }
   const int chunk = 16;
+  static_assert(16 % MS_RING == 0, "a chunk leaves no update pending");
   int done_iters = 0;
   // one chunk of iterations for every right-hand side; all its launches take
   // their scalars from device memory, so the same sequence can be replayed
@@ -290,8 +305,11 @@ int mshift_device(Ctx* c, const yh_inv_par* par, int nrhs, int num, const double
       }
       for (int j = 0; j < nrhs && !e; j++) {
         Rhs& R = rh[j];
-        if ((e = ms_x(c, st + j, mf + j, R.r, R.q))) break;
-        e = ms_k(c, st + j, mf + j, R.r, R.p);
+        const int slot = i % MS_RING;
+        Field* r = R.r[slot];
+        if ((e = ms_x(c, st + j, slot, R.r[(slot + MS_RING - 1) % MS_RING], r, R.q))) break;
+        if ((e = ms_p(c, st + j, r, R.p))) break;
+        if (slot == MS_RING - 1) e = ms_k(c, st + j, mf + j, R.r);
       }
     }
     return e;
