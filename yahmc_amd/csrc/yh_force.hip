@@ -517,14 +517,15 @@ __global__ void __launch_bounds__(128) k_force_logdet(const double2* __restrict_
 //
 // The right-hand link and clover-force matrices reach LDS by direct DMA
 // (global_load_lds, 16 bytes a lane): for column j lane (g, i) fetches the
-// stored element (i, j) into slot word j * 64 + lane, so the stored (r, c)
-// of group g sits at c * 64 + g D + r, and a dagger operand is read
-// transposed and conjugated.  Computed matrices are written the same way.
+// stored element (i, j) into slot word j * 64 + lane (with two rows per lane,
+// a second set of D columns holds the rows i + LPG), so the stored (r, c)
+// of group g sits at FX::word(r, c) past the group's first lane, and a dagger
+// operand is read transposed and conjugated.  Computed matrices are written the same way.
 // Three slots (three LDS objects) rotate.  A step issues the DMAs of later
 // steps (lgkmcnt 0 first, so a slot's earlier reads and writes are done
 // before it is refilled), waits with vmcnt for the DMA of its own slot
 // (vector memory operations complete in issue order; the count is the DMA
-// instructions issued after it, D per matrix, and row loads only add to the
+// instructions issued after it, NDMA per matrix, and row loads only add to the
 // operations after it), and multiplies.  The slot reads are inline asm that
 // completes its own reads, since the compiler would otherwise wait for every
 // outstanding DMA before each one.  The block is one wave: LDS traffic needs
@@ -658,11 +659,25 @@ __global__ void __launch_bounds__(192) k_force_clover_nu(const double* __restric
   project_add<NG, D>(mom, mu, id, g.V, M, coeff, itr);
 }
 
+// Rows per lane: the kernel is bound by its LDS reads (every product reads a
+// whole matrix per lane), so at D_R = 6 a lane holds two rows and uses each
+// element it reads twice.  Three slots (36 KB) leave four one-wave workgroups
+// on a CU, one per SIMD, as its 256 registers do.  Sextet SU(3), 32x24^3: the
+// kernel 6,368 -> 5,902 us under the profiler, the whole end of a fermion
+// force 5,765 -> 5,250 us; three rows a lane (54 KB, two workgroups) 8,199.
+// D_R = 8 keeps one row: two would need 512 registers' worth of rows.
 template <int D>
 struct FX {
-  static constexpr int G = 64 / D;          // groups (x, mu) per wave
-  static constexpr int SLOT = D * 64;       // double2 words per slot
+  static constexpr int RPL = D == 6 ? 2 : 1;  // rows of a matrix per lane
+  static constexpr int LPG = D / RPL;         // lanes of a group: lane i holds rows i, i + LPG, ...
+  static constexpr int G = 64 / LPG;          // groups (x, mu) per wave
+  static constexpr int NDMA = RPL * D;        // DMA instructions (64 words each) per matrix
+  static constexpr int SLOT = NDMA * 64;      // double2 words per slot
+  // word of the stored element (r, c), less the group's first lane
+  static __host__ __device__ constexpr int word(int r, int c) { return ((r / LPG) * D + c) * 64 + r % LPG; }
 };
+template <int D>
+using FxRows = cd[FX<D>::RPL][D];
 
 // step boundary: memory operations stay on their side of it (program order
 // of the issues); the waits are the compiler's own
@@ -692,33 +707,43 @@ __device__ __forceinline__ const double2* fx_clf(const double2* clf, int num, in
 // asynchronous DMA write cannot overtake them
 template <int D>
 __device__ __forceinline__ void fx_dma(double2* slot, const double2* p, int i, size_t stride) {
+  typedef FX<D> F;
   __asm__ volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0) only
   __asm__ volatile("" ::: "memory");
-  const double2* q = p + (size_t)(i * D) * stride;
 #pragma unroll
-  for (int j = 0; j < D; j++) {
-    __attribute__((address_space(3))) void* dst = (__attribute__((address_space(3))) void*)(slot + j * 64);
-    __builtin_amdgcn_global_load_lds((const void*)(q + (size_t)j * stride), dst, 16, 0, 0);
+  for (int h = 0; h < F::RPL; h++) {
+    const double2* q = p + (size_t)((h * F::LPG + i) * D) * stride;
+#pragma unroll
+    for (int j = 0; j < D; j++) {
+      __attribute__((address_space(3))) void* dst = (__attribute__((address_space(3))) void*)(slot + (h * D + j) * 64);
+      __builtin_amdgcn_global_load_lds((const void*)(q + (size_t)j * stride), dst, 16, 0, 0);
+    }
   }
 }
 
-// row i of the stored matrix (DAG: of its conjugate transpose) into registers
+// the lane's rows of the stored matrix (DAG: of its conjugate transpose) into registers
 template <int D, bool DAG>
-__device__ __forceinline__ void fx_row(cd (&r)[D], const double2* p, int i, size_t stride) {
-  const double2* q = p + (size_t)(DAG ? i : i * D) * stride;
+__device__ __forceinline__ void fx_row(FxRows<D>& r, const double2* p, int i, size_t stride) {
 #pragma unroll
-  for (int j = 0; j < D; j++) {
-    const double2 v = q[(size_t)(DAG ? j * D : j) * stride];
-    r[j] = DAG ? cd(v.x, -v.y) : cd(v.x, v.y);
+  for (int h = 0; h < FX<D>::RPL; h++) {
+    const int row = h * FX<D>::LPG + i;
+    const double2* q = p + (size_t)(DAG ? row : row * D) * stride;
+#pragma unroll
+    for (int j = 0; j < D; j++) {
+      const double2 v = q[(size_t)(DAG ? j * D : j) * stride];
+      r[h][j] = DAG ? cd(v.x, -v.y) : cd(v.x, v.y);
+    }
   }
 }
 
-// row i of a register matrix into a slot (stored layout)
+// the lane's rows of a register matrix into a slot (stored layout)
 template <int D>
-__device__ __forceinline__ void fx_put(double2* slot, const cd (&r)[D], int lane) {
+__device__ __forceinline__ void fx_put(double2* slot, const FxRows<D>& r, int lane) {
 #pragma unroll
-  for (int j = 0; j < D; j++) slot[j * 64 + lane] = make_double2(r[j].re, r[j].im);
+  for (int h = 0; h < FX<D>::RPL; h++)
+#pragma unroll
+    for (int j = 0; j < D; j++) slot[(h * D + j) * 64 + lane] = make_double2(r[h][j].re, r[h][j].im);
 }
 
 // LDS reads of the clover-force kernel's slots, written as inline asm so
@@ -821,42 +846,45 @@ __device__ __forceinline__ void fx_rd(fx_d2 (&v)[16], unsigned a) {
 }
 
 // byte offset of element (k, j) of the group's matrix B in a slot, from the
-// group's base: stored (k, j) at word j * 64 + k, or for B = stored^+ the
-// stored (j, k) at word k * 64 + j
-template <bool DAG>
-__host__ __device__ constexpr int fx_off(int k, int j) { return DAG ? k * 1024 + j * 16 : j * 1024 + k * 16; }
+// group's base: the stored (k, j), or for B = stored^+ the stored (j, k)
+template <int D, bool DAG>
+__host__ __device__ constexpr int fx_off(int k, int j) { return 16 * (DAG ? FX<D>::word(j, k) : FX<D>::word(k, j)); }
 
 template <int D, bool DAG, int K0, int NK, size_t... I>
 __device__ __forceinline__ void fx_rd_rows(fx_d2 (&v)[NK * D], unsigned a, std::index_sequence<I...>) {
-  fx_rd<fx_off<DAG>(K0 + (int)I / D, (int)I % D)...>(v, a);
+  fx_rd<fx_off<D, DAG>(K0 + (int)I / D, (int)I % D)...>(v, a);
 }
 
 // out (+)= s (r B), B the group's matrix in a slot (DAG: B = stored^+),
-// `a` the LDS byte address of the slot plus 16 g D; out and r are different
-// arrays.  B is read two rows at a time.
+// `a` the LDS byte address of the slot plus 16 bytes per lane before the
+// group's first; out and r are different arrays.  B is read two rows at a
+// time, each element once for the RPL rows of the lane.
 template <int D, bool DAG, bool ACC, int K0 = 0>
-__device__ __forceinline__ void fx_vm(cd (&out)[D], cd (&r)[D], unsigned a, double s) {
+__device__ __forceinline__ void fx_vm(FxRows<D>& out, FxRows<D>& r, unsigned a, double s) {
   if constexpr (K0 < D) {
     constexpr int NK = (D - K0 >= 2 && D != 8) ? 2 : 1;
     fx_d2 v[NK * D];
     fx_rd_rows<D, DAG, K0, NK>(v, a, std::make_index_sequence<NK * D>{});
 #pragma unroll
-    for (int dk = 0; dk < NK; dk++) {
-      const int k = K0 + dk;
-      const cd rk = s * r[k];
+    for (int dk = 0; dk < NK; dk++)
 #pragma unroll
-      for (int j = 0; j < D; j++) {
-        const fx_d2 m = v[dk * D + j];
-        const double mi = DAG ? -m.y : m.y;
-        // out += rk m as four fused multiply-adds
-        double re = (!ACC && k == 0) ? 0.0 : out[j].re, im = (!ACC && k == 0) ? 0.0 : out[j].im;
-        re = __builtin_fma(rk.re, m.x, re);
-        re = __builtin_fma(-rk.im, mi, re);
-        im = __builtin_fma(rk.re, mi, im);
-        im = __builtin_fma(rk.im, m.x, im);
-        out[j] = cd(re, im);
+      for (int h = 0; h < FX<D>::RPL; h++) {
+        const int k = K0 + dk;
+        const cd rk = s * r[h][k];
+#pragma unroll
+        for (int j = 0; j < D; j++) {
+          const fx_d2 m = v[dk * D + j];
+          const double mi = DAG ? -m.y : m.y;
+          // out += rk m as four fused multiply-adds
+          cd& o = out[h][j];
+          double re = (!ACC && k == 0) ? 0.0 : o.re, im = (!ACC && k == 0) ? 0.0 : o.im;
+          re = __builtin_fma(rk.re, m.x, re);
+          re = __builtin_fma(-rk.im, mi, re);
+          im = __builtin_fma(rk.re, mi, im);
+          im = __builtin_fma(rk.im, m.x, im);
+          o = cd(re, im);
+        }
       }
-    }
     fx_vm<D, DAG, ACC, K0 + NK>(out, r, a, s);
   }
 }
@@ -905,9 +933,9 @@ __global__ void __launch_bounds__(64) k_force_clover_x(const double2* __restrict
   __shared__ __align__(16) double2 sl0[F::SLOT], sl1[F::SLOT], sl2[F::SLOT];
   double2* const sl[3] = {sl0, sl1, sl2};
   const int lane = threadIdx.x;
-  const int gi = min(lane / D, F::G - 1);
-  const int i = lane % D;
-  const int gD = gi * D;
+  const int gi = min(lane / F::LPG, F::G - 1);
+  const int i = lane % F::LPG;
+  const int gD = gi * F::LPG;
   const unsigned a0 = fx_lds(sl0) + 16 * gD, a1 = fx_lds(sl1) + 16 * gD, a2 = fx_lds(sl2) + 16 * gD;
   // work item: (site block, mu), from a 2D grid (order < 0) or a 1D grid
   // with mu fastest, remapped so that each XCD takes runs of `order` items
@@ -915,18 +943,20 @@ __global__ void __launch_bounds__(64) k_force_clover_x(const double2* __restrict
   if (order < 0) { sb = blockIdx.x; mu = blockIdx.y; }
   else { const int b = xcd_block(gridDim.x, order); sb = b >> 2; mu = b & 3; }
   const int grp = sb * F::G + gi;
-  const bool on = lane < F::G * D && grp < g.V;
+  const bool on = lane < F::G * F::LPG && grp < g.V;
   const int id = grp < g.V ? grp : g.V - 1;  // tail lanes compute on a valid site and write nothing
   const size_t SL = g.VHpad, SZ = g.V;
   int c[4], c1[4];
   fcoords(id, g, c);
   const int o1 = fx_nb(c, mu, 1, g, c1);  // x + mu
-  cd Ft[D], S[D], W8[D], W7[D], Q[D], T[D], A[D];
+  FxRows<D> Ft, S, W8, W7, Q, T, A;
 #pragma unroll
-  for (int j = 0; j < D; j++) Ft[j] = cd(0, 0);
+  for (int h = 0; h < F::RPL; h++)
+#pragma unroll
+    for (int j = 0; j < D; j++) Ft[h][j] = cd(0, 0);
   // Each step issues DMAs for later steps (in the order they are needed),
   // waits for the DMA of its own slot by counting the DMA instructions
-  // issued after it (D per matrix), and multiplies.  The row operands are
+  // issued after it (NDMA per matrix), and multiplies.  The row operands are
   // ordinary loads the compiler waits for.
   // prologue: W3 = U(x + nu, mu)^+ and the row of W2 = U(x + mu, nu) for the first nu
   {
@@ -953,11 +983,11 @@ __global__ void __launch_bounds__(64) k_force_clover_x(const double2* __restrict
     // W7 = W2 W3                                (A: row of W2; W3 in s0)
     fx_dma<D>(sl[1], fx_clf<D>(clf, num, fx_opq(o5), g), fx_opq(i), SZ);  // Z4
     fx_dma<D>(sl[2], fx_clf<D>(clf, num, fx_opq(o2), g), fx_opq(i), SZ);  // Z5
-    fx_vmcnt<2 * D>();                                                      // W3
+    fx_vmcnt<2 * F::NDMA>();                                                      // W3
     fx_vm<D, true, false>(W7, A, a0, s2 * s3);
     fx_wait();
     // T = W2 Z4                                                  Z4 s1
-    fx_vmcnt<D>();
+    fx_vmcnt<F::NDMA>();
     fx_vm<D, false, false>(T, A, a1, s2);
     fx_wait();
     // Q = T W3                                                   W3 s0
@@ -967,19 +997,19 @@ __global__ void __launch_bounds__(64) k_force_clover_x(const double2* __restrict
     // Q += W7 Z5                                                 Z5 s2
     fx_dma<D>(sl[0], fx_link<D>(links, fx_opq(o3), nu, g), fx_opq(i), SL);  // W1
     fx_row<D, true>(A, fx_link<D>(links, fx_opq(o3), mu, g), fx_opq(i), SL);  // W0
-    fx_vmcnt<2 * D>();
+    fx_vmcnt<2 * F::NDMA>();
     fx_vm<D, false, true>(Q, W7, a2, 1.0);
     fx_wait();
     // F += sign Q W4                                             W4 s1
     fx_dma<D>(sl[2], fx_clf<D>(clf, num, fx_opq(o3), g), fx_opq(i), SZ);  // Z2
-    fx_vmcnt<2 * D>();
+    fx_vmcnt<2 * F::NDMA>();
     fx_vm<D, true, true>(Ft, Q, a1, sign * s4);
     fx_wait();
     // W8 = W7 W4                                                 W4 s1
     fx_vm<D, true, false>(W8, W7, a1, s4);
     fx_wait();
     // W6 = W0 W1 (in T)                                          W1 s0
-    fx_vmcnt<D>();
+    fx_vmcnt<F::NDMA>();
     fx_vm<D, false, false>(T, A, a0, s0 * s1);
     fx_wait();
     // T1 = W0 Z2 (in T), W6 -> s1                                Z2 s2
@@ -1025,7 +1055,7 @@ __global__ void __launch_bounds__(64) k_force_clover_x(const double2* __restrict
     fx_wait();
   }
   // M = U(x, mu) F, then the projection sum_{k,r} Re (iT_q)_{k r} M_{r k}
-  // with lane i of the group taking q = i, i + D, ...
+  // with lane i of the group taking q = i, i + LPG, ...
   fx_put<D>(sl[2], Ft, lane);
   fx_wait();
   fx_vm<D, false, false>(T, A, a2, fx_sgn(c, mu, g));
@@ -1033,7 +1063,7 @@ __global__ void __launch_bounds__(64) k_force_clover_x(const double2* __restrict
   fx_wait();
   const double f = -coeff * 0.5;
 #pragma unroll
-  for (int q0 = 0; q0 < NG; q0 += D) {
+  for (int q0 = 0; q0 < NG; q0 += F::LPG) {
     const int q = q0 + i;
     if (q < NG) {
       double re = 0.0;
@@ -1042,7 +1072,7 @@ __global__ void __launch_bounds__(64) k_force_clover_x(const double2* __restrict
 #pragma unroll
         for (int r = 0; r < D; r++) {
           const double2 tg = itr[(q * D + k) * D + r];
-          const double2 m = sl0[k * 64 + gD + r];
+          const double2 m = sl0[F::word(r, k) + gD];
           re += tg.x * m.x - tg.y * m.y;
         }
       if (on) mom[(size_t)(mu * NG + q) * g.V + id] += f * re;
@@ -1179,7 +1209,7 @@ int force_clover_core(Ctx* c, double dt) {
         hipLaunchKernelGGL((k_force_clover_nu<NG_, D_>), dim3((c->g.VH + 63) / 64 * 8), dim3(192), 0, c->stream,
                            (const double*)c->clf, links, c->mom, coeff, c->g, c->tab_itr);
       } else {
-        const int groups = 64 / D_;
+        const int groups = FX<D_>::G;
         const unsigned nsb = (unsigned)((c->g.V + groups - 1) / groups);
         dim3 grid = c->force_order < 0 ? dim3(nsb, 4) : dim3(4 * nsb);
         hipLaunchKernelGGL((k_force_clover_x<NG_, D_>), grid, dim3(64), 0, c->stream, (const double2*)c->clf, links,
