@@ -296,8 +296,12 @@ constexpr int hop_min_waves() {
 // again by the time of the 16-bit mixed CG at 32^4, which runs the
 // clover-epilogue variants: t x|y|z 0.2203-0.2210 s against 0.2221-0.2226 s
 // for txy|z (one group 0.2394, t|x y|z 0.2251, one per direction 0.2246).
+// FP64-18 with the clover blocks one after the other as well (bit 5), swept
+// by the CG iteration at 32^4 with its clover inverse staged: t x|y|z 1,017 us,
+// t|x y|z 1,020; without bit 5 1,019; with the epilogue loads after the hop
+// (bit 4, half the registers and twice the waves) 1,065.
 #ifndef YH_SCHED_F64_18
-#define YH_SCHED_F64_18 5
+#define YH_SCHED_F64_18 38
 #endif
 #ifndef YH_SCHED_F64_12
 #define YH_SCHED_F64_12 7
@@ -1085,10 +1089,10 @@ static int hop_dispatch_epi(Ctx* c, const HopArgs& a, int epi, hipStream_t st) {
     // LDS-staged y / z neighbours (yh_tune YH_TUNE_HOP_STAGE) where the
     // geometry allows it (Stage::usable; the kernel has a barrier)
     const size_t lb = Stage<PREC, D>::bytes(c->g);
-    // FP64 clover epilogues run one wave per SIMD (256 VGPRs) and measured
-    // slower staged (H^2 at 32^4: 880 against 859 us); only the plain FP64
-    // hop is staged (134 against 141 us)
-    const bool stage_epi = PREC != PREC_F64 || epi == EPI_PLAIN;
+    // the FP64 clover epilogue runs one wave per SIMD (256 VGPRs) and measured
+    // slower staged (CG iteration at 32^4: 1,055 against 1,024 us); the plain
+    // hop (134 against 141 us) and the clover inverse (1,020 us) are staged
+    const bool stage_epi = PREC != PREC_F64 || epi != EPI_CLOV;
     if (((c->hop_stage >> PREC) & 1) && stage_epi && Stage<PREC, D>::usable(c->g)) {
       switch (epi) {
         case EPI_PLAIN: hipLaunchKernelGGL((k_hop<D, PREC, RECON, EPI_PLAIN, true>), grid, block, lb, st, a); break;
