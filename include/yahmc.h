@@ -428,15 +428,19 @@ int yh_synchronize(yh_ctx* ctx);
  * kernels (D_R <= 3) copy the window of input spinors their y / z
  * neighbours come from into LDS once per workgroup and read those
  * neighbours there (when a (t, x) plane holds a multiple of 256 sites);
- * default 3: FP64 and FP32.  Setting it selects kernels of one thread per
- * site at every size (by default small lattices, up to 32,768 sites a
- * parity, put a site's eight directions on eight waves) */
+ * default 3: FP64 and FP32.  For the kernels of one thread per site
+ * (YH_TUNE_HOP_SPLIT) */
 #define YH_TUNE_HOP_STAGE 8
 /* order in which the clover-force kernel's workgroups take their (site
  * block, mu) work: -1 = all sites of one mu after another; q >= 0 = the
  * four mu of a site block together, in runs of q workgroups per XCD
  * (0, default = one contiguous slab of the lattice per XCD) */
 #define YH_TUNE_FORCE_ORDER 9
+/* 1 (default): on small lattices (up to 32,768 sites a parity, D_R <= 6) the
+ * hop puts a site's eight directions on eight waves; 0: one thread per site
+ * at every size.  The multi-RHS hop, D_R = 8 and hops with a side output
+ * (Dphi and Hphi of a caller's field) take one thread per site either way */
+#define YH_TUNE_HOP_SPLIT 10
 int yh_tune(yh_ctx* ctx, int key, int value);
 /* autotuner (no counterpart in the reference): times the hop of every
  * precision / reconstruction this context holds for each XCD chunk size

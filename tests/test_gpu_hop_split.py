@@ -1,5 +1,5 @@
-"""Small lattices put a site's eight directions on eight waves; setting
-YH_TUNE_HOP_STAGE selects the kernels of one thread per site.  FP64 and FP32
+"""Small lattices put a site's eight directions on eight waves; with
+YH_TUNE_HOP_SPLIT off they take the kernels of one thread per site.  FP64 and FP32
 operators must agree bit for bit (the same sums in the same order), the 16-bit
 ones to the rounding of one multiplication before the fixed-point store, and
 FP64 must meet the oracle; half volumes below, at and past a workgroup of 64
@@ -36,7 +36,7 @@ def test_split_hop_matches_one_thread_per_site(model, dims, bc):
             lat.Hphi_sq(mass, fd, fs)
             outs.append(fd.download()[: o.VH])
             got[split, prec] = outs
-        lat.tune(yh.TUNE_HOP_STAGE, 0)
+        lat.tune(yh.TUNE_HOP_SPLIT, 0)
     want = np.zeros_like(s)
     o.Hphi_sq(mass, want, s.copy())
     assert rel(got[True, "f64"][2], want[: o.VH]) < 1e-13
@@ -60,6 +60,6 @@ def test_split_solves_match(model):
         it = lat.cg_inverter(lat.inv_par(0.1, 1e-24), x, fb)
         it16, _ = lat.cg_mixed(lat.inv_par(0.1, 1e-24, sloppy="f16", reliable_every=50), y, fb)
         res.append((it, x.download()[: o.VH], it16, y.download()[: o.VH]))
-        lat.tune(yh.TUNE_HOP_STAGE, 0)
+        lat.tune(yh.TUNE_HOP_SPLIT, 0)
     assert abs(res[0][0] - res[1][0]) <= 1 and rel(res[0][1], res[1][1]) < 1e-11
     assert abs(res[0][2] - res[1][2]) <= 4 and rel(res[0][3], res[1][3]) < 1e-11

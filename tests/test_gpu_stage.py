@@ -4,7 +4,8 @@ The staged kernels copy the window of input spinors a workgroup's y and z
 neighbours come from (plus the two y-wrap rows of its (t, x) plane) into
 LDS and read those neighbours there; the arithmetic is unchanged, so every
 operator must equal the unstaged one bit for bit, and the oracle's to the
-FP64 bar.  Lattices with a (t, x) plane of a multiple of 256 sites, where
+FP64 bar.  They are kernels of one thread per site, which lattices of this
+size take with YH_TUNE_HOP_SPLIT off.  Lattices with a (t, x) plane of a multiple of 256 sites, where
 the staged kernels run: L_Z = 32 (window halo 17) and L_Z = 64 (halo 33)."""
 import numpy as np
 import pytest
@@ -23,6 +24,7 @@ def test_staged_hop_matches_unstaged_and_oracle(model, dims, bc):
     o, lat, rng = setup(model, dims=dims, bc=bc, csw=1.0, cf=1.1)
     mass = -0.75
     s = src_field(o, rng)
+    lat.tune(yh.TUNE_HOP_SPLIT, 0)
     # FP64 against the oracle, staged
     lat.tune(yh.TUNE_HOP_STAGE, 7)
     fs, fd = lat.field("f64").upload(s), lat.field("f64")
@@ -58,6 +60,7 @@ def test_staged_hop_matches_unstaged_and_oracle(model, dims, bc):
 
 def test_staged_cg_matches_unstaged():
     o, lat, rng = setup("su3_fund", dims=(4, 4, 16, 32), bc=BC_ANTIPERIODIC)
+    lat.tune(yh.TUNE_HOP_SPLIT, 0)
     s = src_field(o, rng, even_only=True)
     fb = lat.field("f64").upload(s)
     sols = []

@@ -1,0 +1,79 @@
+"""Host logic of the C ABI without a GPU: which kernels a call launches, with
+which grid and arguments, and how much device memory it takes, read from a HIP
+runtime that only records (hip_stub.c).  Each case runs in a process of its
+own, which loads that runtime before libyahmc.so."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+LIB = os.path.join(ROOT, "yahmc_amd", "lib", "libyahmc.so")
+pytestmark = pytest.mark.skipif(not os.path.exists(LIB), reason="libyahmc.so not built")
+
+PRELUDE = """
+import ctypes, json, re, sys
+sys.path.insert(0, {root!r})
+stub = ctypes.CDLL({stub!r}, ctypes.RTLD_GLOBAL)
+stub.stub_name.restype = ctypes.c_char_p
+stub.stub_in_use.restype = stub.stub_peak.restype = ctypes.c_size_t
+import numpy as np
+import yahmc_amd as yh
+
+def lattice(dims, nc=3, repr="fundamental"):
+    lat = yh.Lattice(dims, nc=nc, repr=repr)
+    lat.set_gauge(np.zeros((4 * lat.V, 2 * nc * nc)))
+    return lat
+
+def launches(f):
+    "[kernel, grid, watched argument] of every launch of f()"
+    stub.stub_reset()
+    f()
+    out = []
+    for i in range(stub.stub_launches()):
+        g = (ctypes.c_uint32 * 3)()
+        stub.stub_grid(i, g)
+        name = re.match(r"_ZN2yh\\d+(k_[a-z0-9_]+?)(?:I|E|P|R|K|$)", stub.stub_name(i).decode()).group(1)
+        out.append([name, list(g), stub.stub_arg(i)])
+    return out
+
+def names(f):
+    return sorted({{n for n, _, _ in launches(f)}})
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("hip") / "hip_stub.so")
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", so, os.path.join(HERE, "hip_stub.c")], check=True)
+    return so
+
+
+def run(stub, body):
+    """what `body` prints last, as JSON"""
+    out = subprocess.run([sys.executable, "-c", PRELUDE.format(root=ROOT, stub=stub) + body], capture_output=True,
+                         text=True, timeout=120)
+    assert out.returncode == 0, out.stdout + out.stderr
+    return json.loads(out.stdout.splitlines()[-1])
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32", "f16"])
+def test_split_hop_has_a_key_of_its_own(stub, prec):
+    """Setting the staging mask, to its default or to another value, does not
+    change which kernels a small lattice runs; YH_TUNE_HOP_SPLIT does, both ways."""
+    got = run(stub, f"""
+lat = lattice((8, 4, 4, 4))
+s, d = lat.field({prec!r}), lat.field({prec!r})
+hop = lambda: names(lambda: lat.Dphi_eo(d, s))
+out = [hop()]
+for key, value in ((yh.TUNE_HOP_STAGE, 3), (yh.TUNE_HOP_STAGE, 0), (yh.TUNE_HOP_SPLIT, 0), (yh.TUNE_HOP_STAGE, 7),
+                   (yh.TUNE_HOP_SPLIT, 1)):
+    lat.tune(key, value)
+    out.append(hop())
+print(json.dumps(out))
+""")
+    split, one = ["k_hop_split"], ["k_hop"]
+    assert got == [split, split, split, one, one, split]

@@ -23,6 +23,7 @@ TUNE_XCD_CHUNK, TUNE_NET_PREFETCH, TUNE_GRAPHS, TUNE_HALF_LINKS, TUNE_RECON12_F6
 TUNE_LEARNED_GCR = 7
 TUNE_HOP_STAGE = 8
 TUNE_FORCE_ORDER = 9
+TUNE_HOP_SPLIT = 10
 ERRORS = {-1: "invalid argument", -2: "HIP error", -3: "bad state", -4: "not converged", -5: "non-finite",
           -6: "unsupported"}
 

@@ -105,7 +105,7 @@ struct Ctx {
   // read y / z neighbours from an LDS-staged window
   int hop_stage = (1 << PREC_F64) | (1 << PREC_F32);
   // small lattices run a site's directions on eight waves (k_hop_split)
-  int hop_split = 1;
+  int hop_split = 1;  // YH_TUNE_HOP_SPLIT
   int force_order = 0;  // YH_TUNE_FORCE_ORDER
   // solver chunks are captured once into a HIP graph and replayed
   int use_graphs = 1;
