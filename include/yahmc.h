@@ -400,7 +400,8 @@ int yh_bench_copy(yh_ctx* ctx, long bytes, int reps, double* ms);
 int yh_synchronize(yh_ctx* ctx);
 /* tuning knobs of the kernels (no counterpart in the reference):
  * YH_TUNE_XCD_CHUNK = consecutive workgroups each XCD takes (0 = one slab
- * per XCD; default 1/8 of a t-slice) */
+ * per XCD; default 1/8 of a t-slice), in the hops of one thread per site
+ * (YH_TUNE_HOP_SPLIT) */
 #define YH_TUNE_XCD_CHUNK 1
 /* YH_TUNE_NET_PREFETCH = network layer kernels issue the next path's loads
  * before the current path's arithmetic (1) or not (0, default: the extra
@@ -442,10 +443,11 @@ int yh_synchronize(yh_ctx* ctx);
  * (Dphi and Hphi of a caller's field) take one thread per site either way */
 #define YH_TUNE_HOP_SPLIT 10
 int yh_tune(yh_ctx* ctx, int key, int value);
-/* autotuner (no counterpart in the reference): times the hop of every
- * precision / reconstruction this context holds for each XCD chunk size
- * (`reps` launches each) and keeps the fastest per variant; chosen[6]
- * (optional) receives them, index prec * 2 + recon (-1: variant absent) */
+/* autotuner (no counterpart in the reference): times the hop (one thread per
+ * site) of every precision / reconstruction this context holds for each XCD
+ * chunk size (`reps` launches each) and keeps the fastest per variant;
+ * chosen[6] (optional) receives them, index prec * 2 + recon (-1: variant
+ * absent) */
 int yh_autotune(yh_ctx* ctx, int reps, int* chosen);
 
 #ifdef __cplusplus

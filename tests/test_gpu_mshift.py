@@ -143,9 +143,11 @@ def test_graph_replay_matches_eager():
 
 def test_autotune_keeps_results():
     """The autotuner only changes the workgroup -> XCD order: the hop output
-    is bit-identical before and after, and every chunk it picks is valid."""
+    is bit-identical before and after, and every chunk it picks is valid.
+    The hop of one thread per site, which reads the chunk."""
     print("\n[case] autotune", flush=True)
     o, lat, rng = setup("su3_fund", 3, "fundamental", (8, 8, 8, 8), seed=23)
+    lat.tune(yh.TUNE_HOP_SPLIT, 0)
     s = gaussian_spinor(rng, o.V, 3)
     s[: o.VH] = 0
     fs = lat.field("f64").upload(s)

@@ -77,3 +77,18 @@ print(json.dumps(out))
 """)
     split, one = ["k_hop_split"], ["k_hop"]
     assert got == [split, split, split, one, one, split]
+
+
+def test_autotune_times_the_kernels_that_read_the_chunk(stub):
+    """On a small lattice the autotuner times the hop of one thread per site,
+    whose block order the chunk sets, and leaves the eight-wave hop in use."""
+    got = run(stub, """
+lat = lattice((8, 8, 8, 8))
+s, d = lat.field("f64"), lat.field("f64")
+tuned = names(lambda: lat.autotune(reps=1))
+after = names(lambda: lat.Dphi_eo(d, s))
+lat.tune(yh.TUNE_HOP_SPLIT, 0)
+lat.autotune(reps=1)
+print(json.dumps([tuned, after, names(lambda: lat.Dphi_eo(d, s))]))
+""")
+    assert got == [["k_hop"], ["k_hop_split"], ["k_hop"]]

@@ -749,11 +749,20 @@ int yh_bench_hop(yh_ctx* c, int prec, int recon, int reps, yh_field* d, const yh
 // Online autotuner: for every hop variant this context can run, time the
 // plain hop over the even sites for a set of XCD chunk sizes and keep the
 // fastest (the block -> XCD tiling is the shape that matters for this
-// HBM-bound stencil: it sets which t-slices share an XCD's L2).
+// HBM-bound stencil: it sets which t-slices share an XCD's L2).  The kernel
+// timed is the one of one thread per site at every size: the eight-wave hop
+// of small lattices has no chunk, but hops with a side output and the
+// multi-RHS hop of such a lattice take the chosen one.
 int yh_autotune(yh_ctx* c, int reps, int* chosen) {
   if (!c || reps < 1) { set_error("bad argument"); return YH_ERR_ARG; }
   if (!c->gauge_set) { set_error("no gauge field"); return YH_ERR_STATE; }
   YH_HIP(hipSetDevice(c->device));
+  struct SplitOff {
+    Ctx* c;
+    int was;
+    ~SplitOff() { c->hop_split = was; }
+  } split_off = {c, c->hop_split};
+  c->hop_split = 0;
   const int nblocks = (c->g.VH + 255) / 256;
   std::vector<int> cand = {0};
   for (int q = 1; 8 * q <= nblocks; q *= 2) cand.push_back(q);
