@@ -434,8 +434,9 @@ int yh_synchronize(yh_ctx* ctx);
 #define YH_TUNE_HOP_STAGE 8
 /* order in which the clover-force kernel's workgroups take their (site
  * block, mu) work: -1 = all sites of one mu after another; q >= 0 = the
- * four mu of a site block together, in runs of q workgroups per XCD
- * (0, default = one contiguous slab of the lattice per XCD) */
+ * four mu of a site block together, in runs of q workgroups per XCD (0 =
+ * one contiguous slab of the lattice per XCD); default 64 up to D_R = 4,
+ * 0 above */
 #define YH_TUNE_FORCE_ORDER 9
 /* 1 (default): on small lattices (up to 32,768 sites a parity, D_R <= 6) the
  * hop puts a site's eight directions on eight waves; 0: one thread per site

@@ -69,22 +69,24 @@ def test_hmc_force_sequence(model, csw, bc):
     assert rel(lat.get_momenta() - mom0, o.get_momenta() - mom0) < 1e-12
 
 
-def test_clover_force_core_work_orders_agree():
+@pytest.mark.parametrize("model,dims", [("su3_sym", (4, 4, 4, 8)), ("su3_fund", (4, 2, 6, 6)),
+                                        ("su2_fund", (8, 8, 8, 8))])
+def test_clover_force_core_work_orders_agree(model, dims):
     """The clover-force core gives the same momenta (bit for bit) whichever
     order its workgroups take the (site block, mu) items in."""
-    print("\n[case] clover-force core work orders", flush=True)
-    nc, rep = MODELS["su3_sym"]
-    dims = (4, 4, 4, 8)
+    print(f"\n[case] clover-force core work orders {model} {dims}", flush=True)
+    nc, rep = MODELS[model]
     lat = yh.Lattice(dims, nc=nc, repr=rep, bc="antiperiodic", csw=1.0)
     rng = np.random.default_rng(11)
     V = lat.V
     lat.set_gauge(random_gauge(rng, V, nc))
-    a = lat.field("f64").upload(gaussian_spinor(rng, V, 6))
-    b = lat.field("f64").upload(gaussian_spinor(rng, V, 6))
+    a = lat.field("f64").upload(gaussian_spinor(rng, V, lat.dr))
+    b = lat.field("f64").upload(gaussian_spinor(rng, V, lat.dr))
     mom0 = rng.normal(size=(4 * V, nc * nc - 1))
     out = []
-    for order in (-1, 0, 1, 4):
-        lat.tune(yh.TUNE_FORCE_ORDER, order)
+    for order in (None, -1, 0, 1, 4):
+        if order is not None:  # None: the kernel's own
+            lat.tune(yh.TUNE_FORCE_ORDER, order)
         lat.set_momenta(mom0)
         lat.begin_fermion_force()
         lat.clover_fermion_force(1.0, a, b)

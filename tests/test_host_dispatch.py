@@ -92,3 +92,23 @@ lat.autotune(reps=1)
 print(json.dumps([tuned, after, names(lambda: lat.Dphi_eo(d, s))]))
 """)
     assert got == [["k_hop"], ["k_hop_split"], ["k_hop"]]
+
+
+@pytest.mark.parametrize("nc,rep,own", [(3, "fundamental", 64), (2, "fundamental", 64), (3, "symmetric", 0)])
+def test_force_order_reaches_every_clover_force_kernel(stub, nc, rep, own):
+    """YH_TUNE_FORCE_ORDER sets the grid (four rows for -1) and the run length,
+    the last argument, of the clover-force kernel of every representation."""
+    body = f"""
+lat = lattice((8, 4, 4, 4), {nc}, {rep!r})
+lat.set_momenta(np.zeros((4 * lat.V, lat.ng)))
+def core():
+    lat.begin_fermion_force()
+    return [[g[1], a] for n, g, a in launches(lambda: lat.end_fermion_force(0.1)) if "k_force_clover" in n]
+out = [core()]
+for order in (0, 5, -1):
+    lat.tune(yh.TUNE_FORCE_ORDER, order)
+    out.append(core())
+print(json.dumps(out))
+"""
+    assert [o[0][0] for o in run(stub, body)] == [1, 1, 1, 4]
+    assert run(stub, 'stub.stub_watch(b"k_force_clover_", 6)' + body) == [[[1, own]], [[1, 0]], [[1, 5]], [[4, -1]]]

@@ -581,13 +581,18 @@ __device__ __forceinline__ int settled(cd (&m)[D][D]) {
 template <int NG, int D>
 __global__ void __launch_bounds__(192) k_force_clover_nu(const double* __restrict__ clf,
                                                          const double2* __restrict__ links, double* __restrict__ mom,
-                                                         double coeff, Geom g, const double2* __restrict__ itr) {
+                                                         double coeff, Geom g, const double2* __restrict__ itr,
+                                                         int order) {
   __shared__ double2 ex[2][D * D][64];
-  // mu fastest, then parity, then site blocks; 64 workgroups per XCD in turn
-  const int b = xcd_block(gridDim.x, 64);
-  const int mu = b & 3, p = (b >> 2) & 1;
+  // work item (mu, parity, site block): a 2D grid takes all items of one mu
+  // after another (order < 0), a 1D grid mu fastest, each XCD runs of `order`
+  // workgroups
+  int mu, b;
+  if (order < 0) { b = blockIdx.x; mu = blockIdx.y; }
+  else { const int i = xcd_block(gridDim.x, order); b = i >> 2; mu = i & 3; }
+  const int p = b & 1;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int k = (b >> 3) * 64 + lane;
+  const int k = (b >> 1) * 64 + lane;
   const int kk = min(k, g.VH - 1);  // lanes past the end compute on the last site and write nothing
   const int id = p * g.VH + kk, nu = w + (w >= mu);
   const int hi = max(mu, nu), lo = min(mu, nu), num = hi * (hi - 1) / 2 + lo;
@@ -1206,14 +1211,18 @@ int force_clover_core(Ctx* c, double dt) {
   const double2* links = (const double2*)c->links[PREC_F64][RECON_18];
   YH_FORCE_MODELS(
       if constexpr (D_ <= kClfPacked) {
-        hipLaunchKernelGGL((k_force_clover_nu<NG_, D_>), dim3((c->g.VH + 63) / 64 * 8), dim3(192), 0, c->stream,
-                           (const double*)c->clf, links, c->mom, coeff, c->g, c->tab_itr);
+        const int order = c->force_order == FORCE_ORDER_DEFAULT ? 64 : c->force_order;
+        const unsigned nsb = (unsigned)((c->g.VH + 63) / 64 * 2);
+        const dim3 grid = order < 0 ? dim3(nsb, 4) : dim3(4 * nsb);
+        hipLaunchKernelGGL((k_force_clover_nu<NG_, D_>), grid, dim3(192), 0, c->stream, (const double*)c->clf, links,
+                           c->mom, coeff, c->g, c->tab_itr, order);
       } else {
+        const int order = c->force_order == FORCE_ORDER_DEFAULT ? 0 : c->force_order;
         const int groups = FX<D_>::G;
         const unsigned nsb = (unsigned)((c->g.V + groups - 1) / groups);
-        dim3 grid = c->force_order < 0 ? dim3(nsb, 4) : dim3(4 * nsb);
+        const dim3 grid = order < 0 ? dim3(nsb, 4) : dim3(4 * nsb);
         hipLaunchKernelGGL((k_force_clover_x<NG_, D_>), grid, dim3(64), 0, c->stream, (const double2*)c->clf, links,
-                           c->mom, coeff, c->g, c->tab_itr, c->force_order);
+                           c->mom, coeff, c->g, c->tab_itr, order);
       });
   YH_HIP(hipGetLastError());
   return YH_OK;

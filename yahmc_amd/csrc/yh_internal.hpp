@@ -53,6 +53,8 @@ struct SolverScalars {
   int pad[10];
 };
 
+enum { FORCE_ORDER_DEFAULT = -2 };  // each clover-force kernel's own order
+
 struct Ctx {
   Geom g;
   int nc, dr, repr;
@@ -106,7 +108,7 @@ struct Ctx {
   int hop_stage = (1 << PREC_F64) | (1 << PREC_F32);
   // small lattices run a site's directions on eight waves (k_hop_split)
   int hop_split = 1;  // YH_TUNE_HOP_SPLIT
-  int force_order = 0;  // YH_TUNE_FORCE_ORDER
+  int force_order = FORCE_ORDER_DEFAULT;  // YH_TUNE_FORCE_ORDER
   // solver chunks are captured once into a HIP graph and replayed
   int use_graphs = 1;
   // model tables of this context's (nc, representation), in device memory
