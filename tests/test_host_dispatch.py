@@ -112,3 +112,27 @@ print(json.dumps(out))
 """
     assert [o[0][0] for o in run(stub, body)] == [1, 1, 1, 4]
     assert run(stub, 'stub.stub_watch(b"k_force_clover_", 6)' + body) == [[[1, own]], [[1, 0]], [[1, 5]], [[4, -1]]]
+
+
+@pytest.mark.parametrize("nrhs,num", [(1, 1), (1, 12), (4, 3)])
+def test_multishift_takes_half_fields(stub, nrhs, num):
+    """The multishift's working fields are even or odd halves: four residuals,
+    p, q and a direction per shift, two operator temporaries when batched."""
+    got = run(stub, f"""
+lat = lattice((8, 8, 8, 8))
+srcs = [lat.field("f64") for _ in range({nrhs})]
+dsts = [[lat.field("f64") for _ in range({num})] for _ in srcs]
+def solve():
+    try:
+        lat.cg_mshift_batched(lat.inv_par(0.1, 1e-20, max_iter=16), [0.1] * {num}, dsts, srcs)
+    except yh.YahmcError as e:
+        assert e.code == -4
+solve()  # the context's own temporaries
+before = stub.stub_in_use()
+stub.stub_reset()
+solve()
+half = 64 * lat.dr * ((lat.VH + 63) // 64 * 64 + 64)
+print(json.dumps([(stub.stub_peak() - before) / half, stub.stub_in_use() - before]))
+""")
+    halves = nrhs * (6 + num + (2 if nrhs > 1 else 0))
+    assert halves <= got[0] < halves + 1 and got[1] == 0
