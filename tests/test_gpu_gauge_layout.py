@@ -95,3 +95,24 @@ def test_ragged_fermion_forces(model, nc, rep, dims, bc):
         x.end_fermion_force(0.3)
     got, want = lat.get_momenta(), o.get_momenta()
     assert np.abs(got - want).max() < 1e-12 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("nc,rep,dims", [(2, "fundamental", (34, 26, 26, 26)), (3, "fundamental", (26, 22, 18, 26)),
+                                         (4, "antisymmetric", (14, 18, 26, 22))])
+def test_host_links_in_pieces(nc, rep, dims):
+    """Links of more than 128 MiB cross to the device and back in pieces: these
+    volumes are no multiple of a piece, pieces cross the parity boundary, and
+    so does a block of 16 sites where the half volume is 8 past a multiple."""
+    V = int(np.prod(dims))
+    assert V * 64 * nc * nc > 128 << 20
+    print(f"\n[case] host links in pieces nc={nc} {dims}", flush=True)
+    lat = yh.Lattice(dims, nc=nc, repr=rep, bc="antiperiodic", csw=0.0)
+    rng = np.random.default_rng(73)
+    links = rng.random(size=(4 * V, 2 * nc * nc))  # any numbers: they are only moved
+    lat.set_gauge(links)
+    assert np.array_equal(lat.get_gauge(), links)
+    if rep == "fundamental":
+        # represented links are copies in the same planes, but for the antiperiodic sign of direction 0 at t = 0
+        got = lat.gauge_repr().reshape(V, 4, -1)
+        want = links.reshape(V, 4, -1).copy()
+        assert np.array_equal(got[:, 1:], want[:, 1:]) and np.array_equal(np.abs(got), np.abs(want))

@@ -136,3 +136,15 @@ print(json.dumps([(stub.stub_peak() - before) / half, stub.stub_in_use() - befor
 """)
     halves = nrhs * (6 + num + (2 if nrhs > 1 else 0))
     assert halves <= got[0] < halves + 1 and got[1] == 0
+
+
+@pytest.mark.parametrize("nc", [2, 4])
+def test_links_are_held_once(stub, nc):
+    """A context keeps its fundamental links once; the buffer that their host
+    transfers go through is bounded."""
+    used = run(stub, f"""
+lat = yh.Lattice((64, 48, 48, 48), nc={nc})
+print(json.dumps(stub.stub_in_use()))
+""")
+    V = 64 * 48**3
+    assert used < 64 * nc * nc * V + (144 << 20)

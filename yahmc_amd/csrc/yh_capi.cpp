@@ -406,7 +406,7 @@ int yh_create(const yh_lattice* lat, yh_ctx** out) {
   for (int i = 0; i < Ctx::SC_RING && e == hipSuccess; i++)
     e = hipEventCreateWithFlags(&c->ev_ring[i], hipEventDisableTiming);
   if (e == hipSuccess) e = hipMalloc(&c->fund, sizeof(double2) * 8 * (size_t)c->g.VHpad * lat->nc * lat->nc);
-  if (e == hipSuccess) e = hipMalloc(&c->fund_aos, sizeof(double) * 4 * (size_t)V * 2 * lat->nc * lat->nc);
+  if (e == hipSuccess) e = hipMalloc(&c->fund_stage, fund_stage_bytes(c));
   if (e == hipSuccess) e = hipMalloc(&c->tab, sizeof(double2) * (TAB_BASIS + TAB_ITR));
   if (e != hipSuccess) {
     set_error(std::string("context allocation: ") + hipGetErrorString(e));
@@ -443,7 +443,7 @@ int yh_destroy(yh_ctx* c) {
   for (int i = 4; i < 6; i++)
     if (c->tmp[i]) { (void)hipFree(c->tmp[i]->mem); delete static_cast<yh_field*>(c->tmp[i]); }
   if (c->fund) (void)hipFree(c->fund);
-  if (c->fund_aos) (void)hipFree(c->fund_aos);
+  if (c->fund_stage) (void)hipFree(c->fund_stage);
   if (c->tab) (void)hipFree(c->tab);
   if (c->logdet_site) (void)hipFree(c->logdet_site);
   if (c->mom) (void)hipFree(c->mom);

@@ -53,6 +53,7 @@ struct SolverScalars {
   int pad[10];
 };
 
+enum { FUND_STAGE_BYTES = 128 << 20 };
 enum { FORCE_ORDER_DEFAULT = -2 };  // each clover-force kernel's own order
 
 struct Ctx {
@@ -63,10 +64,10 @@ struct Ctx {
   hipStream_t stream;
   int nblk;            // blocks of 256 threads over one half
   // gauge field: fundamental links, component planes like the represented
-  // links (yh_common.hpp), and the buffer that host transfers in the
-  // reference layout (4V suNg) go through
+  // links (yh_common.hpp), and the buffer (at most FUND_STAGE_BYTES) that host
+  // transfers in the reference layout (4V suNg) go through
   double2* fund = nullptr;
-  double* fund_aos = nullptr;
+  double* fund_stage = nullptr;
   // represented links, SoA, per (prec, recon); null if not built
   void* links[3][2] = {{nullptr, nullptr}, {nullptr, nullptr}, {nullptr, nullptr}};
   // packed clover term (no mass) for both parities, per precision
@@ -143,6 +144,7 @@ int field_convert(Ctx* c, Field* dst, int dpar, const Field* src, int spar);
 int gauge_init_basis(Ctx* c);
 int gauge_upload(Ctx* c, const double* host);    // host links (4V suNg) -> fund
 int gauge_download(Ctx* c, double* host);        // fund -> host links
+size_t fund_stage_bytes(const Ctx* c);           // size of fund_stage
 int gauge_represent(Ctx* c);                 // fund -> represented links, every precision
 int clover_build(Ctx* c);                    // packed clover term, every precision
 int clover_invert(Ctx* c, double sigma);     // odd-site inverses (+ logdet)
