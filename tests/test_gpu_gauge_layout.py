@@ -15,7 +15,7 @@ yh = pytest.importorskip("yahmc_amd")
 # half volumes 8 (less than a wavefront), 144 = 2 * 64 + 16 and 720 = 11 * 64 + 16
 DIMS = [(2, 2, 2, 2), (4, 2, 6, 6), (6, 4, 6, 10)]
 MODELS = [("su2_fund", 2, "fundamental"), ("su3_fund", 3, "fundamental"), ("su3_sym", 3, "symmetric"),
-          ("su4_asym", 4, "antisymmetric")]
+          ("su4_asym", 4, "antisymmetric"), ("su2_adj", 2, "adjoint"), ("su3_adj", 3, "adjoint")]
 
 
 @pytest.mark.parametrize("model,nc,rep", MODELS)
