@@ -24,8 +24,10 @@ MVM_DPHI, MVM_HPHI, MVM_HPHI_SQ = 0, 1, 2
 MODELS = {
     "su3_fund": (3, 0),
     "su2_fund": (2, 0),
+    "su4_fund": (4, 0),
     "su2_adj": (2, 1),
     "su3_adj": (3, 1),
+    "su2_sym": (2, 2),
     "su3_sym": (3, 2),
     "su3_asym": (3, 3),
     "su4_asym": (4, 3),

@@ -19,7 +19,7 @@
  *                                                  (library/geometry.cpp:756-878)
  *
  * Compile-time model, as in the reference (programs/Makefile:6-11):
- *   OR_NC   = number of colours (2 or 3)
+ *   OR_NC   = number of colours (2, 3 or 4)
  *   OR_REPR = 0 fundamental, 1 adjoint, 2 symmetric, 3 antisymmetric
  *             (the reference's REPR_ID values, include/repr.h:9-39)
  * Boundary conditions and c_sw are run-time parameters here.

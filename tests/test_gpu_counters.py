@@ -117,11 +117,13 @@ def test_mvm_count_of_bicgstab_mshift_and_mixed_cg():
     assert lat.mvm_get() == 2 * (1 + it + upd)
 
 
-def test_fp64_12_real_links():
+@pytest.mark.parametrize("split", [1, 0])
+def test_fp64_12_real_links(split):
     """FP64 operators reading 12-real SU(3) links (third row conj(r0 x r1))
     against the oracle's 18-real operator: the reconstruction is exact up to
-    rounding for SU(3) links."""
+    rounding for SU(3) links.  By either hop (YH_TUNE_HOP_SPLIT)."""
     o, lat, rng, _ = setup(dims=(4, 4, 4, 8))
+    lat.tune(yh.TUNE_HOP_SPLIT, split)
     lat.tune(yh.TUNE_RECON12_F64, 1)
     mass = -0.75
     s = even_source(o, rng)

@@ -17,7 +17,7 @@ yh = pytest.importorskip("yahmc_amd")
 
 MODELS = {"su3_fund": (3, "fundamental"), "su2_adj": (2, "adjoint"), "su3_sym": (3, "symmetric"),
           "su2_fund": (2, "fundamental"), "su3_adj": (3, "adjoint"), "su3_asym": (3, "antisymmetric"),
-          "su4_asym": (4, "antisymmetric")}
+          "su4_asym": (4, "antisymmetric"), "su4_fund": (4, "fundamental")}
 BC_NAMES = {BC_PERIODIC: "periodic", BC_ANTIPERIODIC: "antiperiodic", BC_OPEN: "open"}
 
 
@@ -29,7 +29,7 @@ def rel(a, b):
                                           ("su2_adj", 1.2, BC_ANTIPERIODIC), ("su3_sym", 1.0, BC_ANTIPERIODIC),
                                           ("su2_fund", 1.0, BC_PERIODIC), ("su3_adj", 1.0, BC_ANTIPERIODIC),
                                           ("su3_asym", 1.1, BC_PERIODIC), ("su4_asym", 1.0, BC_ANTIPERIODIC),
-                                          ("su3_fund", 1.0, BC_OPEN)])
+                                          ("su3_fund", 1.0, BC_OPEN), ("su4_fund", 1.0, BC_ANTIPERIODIC)])
 def test_hmc_force_sequence(model, csw, bc):
     print(f"\n[case] forces model={model} csw={csw} bc={bc}", flush=True)
     nc, rep = MODELS[model]

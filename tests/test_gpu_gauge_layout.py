@@ -15,7 +15,8 @@ yh = pytest.importorskip("yahmc_amd")
 # half volumes 8 (less than a wavefront), 144 = 2 * 64 + 16 and 720 = 11 * 64 + 16
 DIMS = [(2, 2, 2, 2), (4, 2, 6, 6), (6, 4, 6, 10)]
 MODELS = [("su2_fund", 2, "fundamental"), ("su3_fund", 3, "fundamental"), ("su3_sym", 3, "symmetric"),
-          ("su4_asym", 4, "antisymmetric"), ("su2_adj", 2, "adjoint"), ("su3_adj", 3, "adjoint")]
+          ("su4_asym", 4, "antisymmetric"), ("su2_adj", 2, "adjoint"), ("su3_adj", 3, "adjoint"),
+          ("su4_fund", 4, "fundamental"), ("su2_sym", 2, "symmetric")]
 
 
 @pytest.mark.parametrize("model,nc,rep", MODELS)
@@ -63,7 +64,7 @@ def test_ragged_lattices(model, nc, rep, dims, bc):
 
 
 FORCE_MODELS = [("su2_fund", 2, "fundamental"), ("su3_fund", 3, "fundamental"), ("su4_asym", 4, "antisymmetric"),
-                ("su3_sym", 3, "symmetric")]
+                ("su3_sym", 3, "symmetric"), ("su4_fund", 4, "fundamental"), ("su2_adj", 2, "adjoint")]
 
 
 @pytest.mark.parametrize("model,nc,rep", FORCE_MODELS)

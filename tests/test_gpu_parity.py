@@ -18,7 +18,7 @@ yh = pytest.importorskip("yahmc_amd")
 
 MODELS = {"su3_fund": (3, "fundamental"), "su2_fund": (2, "fundamental"), "su2_adj": (2, "adjoint"),
           "su3_sym": (3, "symmetric"), "su3_asym": (3, "antisymmetric"), "su4_asym": (4, "antisymmetric"),
-          "su3_adj": (3, "adjoint")}
+          "su3_adj": (3, "adjoint"), "su4_fund": (4, "fundamental"), "su2_sym": (2, "symmetric")}
 BCN = {BC_PERIODIC: "periodic", BC_ANTIPERIODIC: "antiperiodic", BC_OPEN: "open", BC_SF: "sf"}
 
 
@@ -95,7 +95,8 @@ def test_clover_apply_and_inverse(bc):
 @pytest.mark.parametrize("model,bc", [("su3_fund", BC_ANTIPERIODIC), ("su3_fund", BC_PERIODIC), ("su3_fund", BC_OPEN),
                                       ("su3_fund", BC_SF), ("su2_fund", BC_ANTIPERIODIC), ("su2_adj", BC_ANTIPERIODIC),
                                       ("su3_sym", BC_ANTIPERIODIC), ("su3_asym", BC_OPEN),
-                                      ("su4_asym", BC_ANTIPERIODIC), ("su3_adj", BC_ANTIPERIODIC), ("su3_adj", BC_OPEN)])
+                                      ("su4_asym", BC_ANTIPERIODIC), ("su3_adj", BC_ANTIPERIODIC), ("su3_adj", BC_OPEN),
+                                      ("su4_fund", BC_ANTIPERIODIC), ("su4_fund", BC_SF), ("su2_sym", BC_OPEN)])
 def test_schur_operators(model, bc):
     o, lat, rng = setup(model, dims=(4, 4, 4, 4), bc=bc, csw=1.0, cf=1.1)
     mass = -0.75
@@ -273,12 +274,15 @@ def test_bicgstab_and_mshift():
         assert rel(x[: o.VH], xo[: o.VH]) < 1e-11
 
 
-def test_half_links_under_fp32_spinors():
+@pytest.mark.parametrize("split", [1, 0])
+def test_half_links_under_fp32_spinors(split):
     """YH_TUNE_HALF_LINKS: the FP32 operator reading FP16 12-real links agrees
     with the oracle to FP16 link accuracy, and the mixed CG built on it still
-    reaches the FP64 true residual."""
+    reaches the FP64 true residual; by the hop of small lattices and by the
+    one of large lattices (YH_TUNE_HOP_SPLIT)."""
     o, lat, rng = setup("su3_fund", dims=(8, 8, 8, 8), bc=BC_ANTIPERIODIC, csw=1.0, seed=32244)
     mass, prec = -0.75, 1e-20
+    lat.tune(yh.TUNE_HOP_SPLIT, split)
     lat.tune(yh.TUNE_HALF_LINKS, 1)
     s = src_field(o, rng, even_only=True)
     want = np.zeros_like(s)
@@ -298,11 +302,14 @@ def test_half_links_under_fp32_spinors():
     assert rel(fd.download()[: o.VH], want[: o.VH]) < 2e-6
 
 
+@pytest.mark.parametrize("split", [1, 0])
 @pytest.mark.parametrize("sloppy", ["f32", "f16"])
-def test_cg_mixed_true_residual(sloppy):
+def test_cg_mixed_true_residual(sloppy, split):
     """Mixed-precision CG reaches the FP64 true residual 1e-10 (prec 1e-20),
-    checked with the oracle's FP64 operator on the returned solution."""
+    checked with the oracle's FP64 operator on the returned solution; by
+    either hop (YH_TUNE_HOP_SPLIT)."""
     o, lat, rng = setup("su3_fund", dims=(8, 8, 8, 8), bc=BC_ANTIPERIODIC, csw=1.0, seed=32244)
+    lat.tune(yh.TUNE_HOP_SPLIT, split)
     mass, prec = -0.75, 1e-20
     b = src_field(o, rng, even_only=True)
     fb = lat.field("f64").upload(b)

@@ -61,7 +61,8 @@ def hmc_force(o, mass, pf, prec=1e-28):
 
 
 @pytest.mark.parametrize("model,csw,bc", [("su3_fund", 1.0, BC_ANTIPERIODIC), ("su3_fund", 0.0, BC_PERIODIC),
-                                          ("su2_adj", 1.3, BC_ANTIPERIODIC), ("su3_sym", 1.0, BC_PERIODIC)])
+                                          ("su2_adj", 1.3, BC_ANTIPERIODIC), ("su3_sym", 1.0, BC_PERIODIC),
+                                          ("su4_fund", 1.0, BC_ANTIPERIODIC)])
 def test_force_is_minus_gradient_of_action(model, csw, bc):
     o = Oracle(model).init((4, 4, 2, 4), bc=bc, csw=csw)
     rng = np.random.default_rng(21)

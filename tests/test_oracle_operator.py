@@ -182,7 +182,7 @@ def test_schur_operator_brute_force():
     assert np.abs(side + Dh[O, E] @ spinor_to_complex(psi, dr).reshape(-1)[:ne]).max() < 1e-13
 
 
-@pytest.mark.parametrize("model", ["su3_fund", "su2_adj", "su3_sym"])
+@pytest.mark.parametrize("model", ["su3_fund", "su4_fund", "su2_adj", "su2_sym", "su3_sym"])
 def test_gamma5_hermiticity(model):
     """<u, H v> = <H u, v> (checks/dirac.cpp:7-51)."""
     o, rng = make(model=model, csw=1.0)

@@ -23,7 +23,8 @@ def R(o, u):
     return mat_to_complex(o.represent_link(complex_to_mat(u[None]).ravel())[None], o.dr)[0]
 
 
-@pytest.mark.parametrize("model", ["su3_fund", "su2_fund", "su2_adj", "su3_adj", "su3_sym", "su3_asym", "su4_asym"])
+@pytest.mark.parametrize("model", ["su3_fund", "su2_fund", "su4_fund", "su2_adj", "su3_adj", "su2_sym", "su3_sym", "su3_asym",
+                                   "su4_asym"])
 def test_homomorphism_and_orthogonality(model):
     o = Oracle(model).init((2, 2, 2, 2))
     rng = np.random.default_rng(3)
@@ -131,7 +132,7 @@ def _ref_adj(U, n):
 
 
 @pytest.mark.parametrize("model,fn", [("su3_sym", _ref_sym), ("su3_asym", _ref_asym), ("su4_asym", _ref_asym),
-                                      ("su2_adj", _ref_adj), ("su3_adj", _ref_adj)])
+                                      ("su2_adj", _ref_adj), ("su3_adj", _ref_adj), ("su2_sym", _ref_sym)])
 def test_matches_reference_entrywise_expansion(model, fn):
     o = Oracle(model).init((2, 2, 2, 2))
     rng = np.random.default_rng(11)
