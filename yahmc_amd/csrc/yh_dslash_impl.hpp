@@ -297,9 +297,19 @@ constexpr int hop_min_waves() {
 // clover-epilogue variants: t x|y|z 0.2203-0.2210 s against 0.2221-0.2226 s
 // for txy|z (one group 0.2394, t|x y|z 0.2251, one per direction 0.2246).
 // FP64-18 with the clover blocks one after the other as well (bit 5), swept
-// by the CG iteration at 32^4 with its clover inverse staged: t x|y|z 1,017 us,
-// t|x y|z 1,020; without bit 5 1,019; with the epilogue loads after the hop
-// (bit 4, half the registers and twice the waves) 1,065.
+// by 96 iterations of the CG, in ms: t x|y|z with bit 5 (38), t|x y|z with it
+// (37), t x|y|z without (6), t|x y|z without (5):
+//                    32x16^3  32x20^3    24^4  48x24^3    32^4
+//   SU(3)        38    12.23    23.81   33.95    67.74   95.82
+//                37    12.22    23.89   34.09    67.84   95.92
+//                 6    12.27    23.93   34.11    68.08   96.47
+//                 5    12.28    24.06   34.32    68.04   96.22
+//   SU(2)        38     7.62    13.44   18.53    37.07   51.59
+//                 5     7.64    13.52   18.49    37.11   51.41
+// (runs of one side differ by up to 0.4 %; SU(2) adjoint as SU(3)): small but of
+// one sign at D_R = 3, even at D_R = 2, which takes the same mask.  With the
+// epilogue loads after the hop (bit 4, half the registers and twice the waves)
+// the iteration at 32^4 takes 1,065 instead of 1,017 us.
 #ifndef YH_SCHED_F64_18
 #define YH_SCHED_F64_18 38
 #endif
@@ -546,16 +556,17 @@ __global__ void __launch_bounds__(YH_HOP_BLOCK, hop_min_waves<PREC>()) k_hop(Hop
 }
 
 // ---------------------------------------------------------------------------
-// Small lattices: a site's eight directions on eight waves (D_R <= 6).  With
-// one thread per site a lattice of up to ~65,000 sites a half keeps at most
-// one wave per SIMD, and the launch lasts as long as one thread's chain of
-// eight neighbour loads and products.  Here a workgroup takes 64 sites and
-// wave w the direction w: it loads one neighbour and one link and leaves the
-// transported half spinor in LDS; waves 0 and 1, which (D_R <= 4,
-// FP32 and 16-bit) have their chiral block of the clover term in flight
-// meanwhile, add the eight in the order of k_hop and finish spins 0, 1 and 2, 3.  FP64 and
-// FP32 results equal k_hop's bit for bit (FP64 norms are summed in another
-// order); 16-bit ones differ by the rounding of one multiplication.
+// Small lattices (split_limit): a site's eight directions on eight waves
+// (D_R <= 6; YH_TUNE_HOP_SPLIT).  With one thread per site a lattice of up to
+// ~65,000 sites a half keeps at most one wave per SIMD, and the launch lasts
+// as long as one thread's chain of eight neighbour loads and products.  Here a
+// workgroup takes 64 sites and wave w the direction w: it loads one neighbour
+// and one link and leaves the transported half spinor in LDS; waves 0 and 1,
+// which have their chiral block of the clover term in flight meanwhile (up to
+// D_R = 3, and D_R = 4 in FP32 and 16-bit), add the eight in the order of k_hop
+// and finish spins 0, 1 and 2, 3.  FP64 and FP32 results equal k_hop's bit for
+// bit (FP64 norms are summed in another order); 16-bit ones differ by the
+// rounding of one multiplication.
 // Not for a call with a side output (aux), which keeps k_hop.
 template <int D, typename R>
 struct SplitArgs {
@@ -835,15 +846,25 @@ __global__ void __launch_bounds__(512) k_hop_split(HopArgs a) {
 }
 
 // largest half volume that k_hop_split takes: two workgroups (64 sites each)
-// per CU.  H^2 through yh_Hphi_sq (three of its four hops split, ~10 us of it
-// the call), split / one thread per site, in us:
-//                   VH 4,096       14,400        32,768        49,152
-//   SU(3) FP64    41.1 /  67.3  51.2 /  81.3  76.8 /  84.1  105.6 /  95.2
-//   SU(3) 16-bit  30.9 /  39.8  32.9 /  42.5  43.5 /  44.0   51.8 /  46.0
-//   SU(4) FP32    39.6 /  54.8  49.2 /  73.0  71.4 /  78.6   96.7 /  88.0
-//   sextet FP64   83.3 / 177.5  114.3 / 195.0  212.2 / 214.3  324.3 / 277.8
-//   SU(2) FP32    28.1 /  34.6  30.2 /  35.9  35.6 /  37.1   44.2 /  40.2
-// D_R = 8 keeps one thread per site (0).
+// per CU, so that the launch is one round of workgroups.  H^2 through
+// yh_Hphi_sq (three of its four hops split, ~10 us of it the call), split / one
+// thread per site, in us:
+//                   VH 8,192       16,384        28,672        32,768
+//   SU(2) FP64    34.6 /  45.1   39.9 /  52.4   46.4 /  56.3   48.8 /  56.7
+//   SU(2) 16-bit  27.1 /  32.6   28.2 /  32.6   32.0 /  32.7   32.4 /  33.3
+//   SU(3) FP64    45.5 /  69.5   55.1 /  76.8   70.3 /  79.8   75.8 /  82.6
+//   SU(3) FP32    32.2 /  42.0   35.2 /  44.6   44.3 /  46.3   45.7 /  47.5
+//   SU(3) 16-bit  31.1 /  41.0   33.8 /  42.5   42.2 /  42.9   42.7 /  42.2
+//   SU(4) FP64    58.4 / 106.6   73.4 / 110.8   96.2 / 117.6  103.7 / 121.2
+//   SU(4) 16-bit  38.1 /  52.4   41.3 /  59.9   54.2 /  62.3   56.8 /  62.9
+//   sextet FP64   90.0 / 182.3  132.7 / 192.7  185.0 / 206.3  213.4 / 214.3
+//   sextet FP32   63.6 /  97.1   75.2 /  99.5  103.7 / 108.4  110.5 / 113.1
+//   sextet 16-bit 61.2 /  90.4   65.6 /  98.6   92.5 / 102.8   95.3 / 104.6
+// One line for all of them: at it the closest (SU(3) 16-bit, sextet FP64) are
+// even, and past it, where a second round begins, every one measured loses (at
+// 49,152 SU(3) FP64 105.6 / 95.2, 16-bit 51.8 / 46.0, SU(4) FP32 96.7 / 88.0,
+// sextet FP64 324.3 / 277.8, SU(2) FP32 44.2 / 40.2).  D_R = 8 keeps one thread
+// per site (0).
 template <int D>
 constexpr int split_limit() {
   return D <= 6 ? 32768 : 0;

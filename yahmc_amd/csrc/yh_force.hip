@@ -353,7 +353,7 @@ __global__ void __launch_bounds__(256) k_force_hop(FF f, const double2* __restri
 // clover force matrices, one thread per site  (forces.cpp:130-168):
 // F = sum_spin (S X) Y^+ + (S Y) X^+ with S = gamma5 sigma anti-Hermitian, so
 // F = M - M^+ with M = sum_spin (S X) Y^+.  Packed matrices (PACK): M once
-// and D^2 reals read and written, 741 -> 240 us at 32^4 for SU(3).
+// and D^2 reals read and written, 741 -> 316 us at 32^4 for SU(3).
 template <int D, bool PACK>
 __global__ void __launch_bounds__(256) k_force_clover_site(FF f, double* __restrict__ clf, double residue, Geom g) {
   int id = blockIdx.x * 256 + threadIdx.x;

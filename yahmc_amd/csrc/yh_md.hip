@@ -445,7 +445,8 @@ __device__ __forceinline__ void project(double (&out)[NC * NC - 1], const M<NC>&
 // of 64 sites, so that the workgroups that share links run side by side; each
 // XCD takes 64 consecutive workgroups in turn, which keeps the time
 // neighbours of its sites closer than one contiguous slab per XCD does
-// (SU(3) Wilson force at 32^4: 690 us, one slab per XCD 746).
+// (SU(3) Wilson force at 32^4, calls back to back: 690 us, one slab per XCD
+// 746).
 struct ForceItem {
   int mu, p, k;  // direction, parity, half index (may lie past the end)
 };
@@ -485,7 +486,8 @@ __device__ __forceinline__ void force_tail(M<NC>& S, const double2* fund, double
 // staples weighted by their plaquettes' weights (forces.cpp:262-283,
 // staples.cpp:82-107).  A workgroup takes 64 consecutive sites of one parity
 // and one mu, one wave per nu.  Bound by the 19 link reads per (x, mu) from
-// L2: 690 us at 32^4 (16.6 TB/s of link reads; 1,614 us with the links as an
+// L2: 728 us at 32^4 among the kernels of a leapfrog step, 690 back to back
+// (15.7 and 16.6 TB/s of link reads; 1,614 us in the step with the links as an
 // array of 144-byte structures, where every load of a wave touches 64 or
 // more cache lines, and one thread per link).  Measured and not kept: one
 // wave per plane forming the plaquettes that serve two links each (fewer
